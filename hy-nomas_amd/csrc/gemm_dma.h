@@ -106,6 +106,15 @@ HN_GEMM_HD TailSrc tail_wide_src(int q, int l, int ar, int64_t m0, int64_t M, in
     return t;
 }
 
+// Work item -> tile of gemm_small_kernel: groups of `group` tile rows walking N
+// (the last group takes the rows left).
+HN_GEMM_HD void small_tile(int item, int tiles_m, int tiles_n, int group, int& tm, int& tn) {
+    const int first = item / (group * tiles_n) * group;
+    const int gm = tiles_m - first < group ? tiles_m - first : group, at = item - first * tiles_n;
+    tm = first + at % gm;
+    tn = at / gm;
+}
+
 // K steps of a tail wave: wave w of SK takes steps w + SK t, t < T =
 // tail_steps(KT, w, SK); loads issued past its last step repeat step T - 1
 // (in bounds, never read), so every step issues the same loads.

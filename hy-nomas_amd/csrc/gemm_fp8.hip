@@ -7,10 +7,12 @@
 // nn.Linear weight layout). Two scale modes:
 //   ROWCOL    per-token x per-output-channel scales, bias and optional
 //             GELU-tanh fused in the epilogue (gemm_rowcol_oe_kernel, a
-//             persistent 4-wave kernel; gemm_rowcol_kernel for short K);
+//             persistent 4-wave kernel);
 //   BLOCKWISE 128x128 block scales on both operands (the decoder contract):
 //             each 128-wide K step is promoted with its own sa * sb factor
 //             (gemm_bw8_kernel, 8 waves).
+// Launches that 256 x 256 tiles would leave uneven or idle, and short K, run
+// smaller tiles in either mode (gemm_small_kernel; small_plan chooses).
 //
 // Tiling: a workgroup owns a 256 x 256 output tile; with 4 waves (2 x 2) each
 // wave owns 128 x 128 = 4 x 4 MFMA blocks of 32 x 32 (256 fp32 accumulators
@@ -22,7 +24,10 @@
 // The MFMA's first operand is the weight tile and its second the activation
 // tile, i.e. the wave computes out^T: each lane then holds four consecutive
 // output columns n..n+3 of one row m and stores them as one 8-byte write.
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
+#include <iterator>
 #include <type_traits>
 
 #include "hn_capi_internal.h"
@@ -34,15 +39,7 @@ namespace gemm {
 
 constexpr int BM = 256, BN = 256, BK = 128;
 constexpr int NT = 256;
-constexpr int TILE_BYTES = BM * BK;         // one operand tile, 32 KB
-constexpr int STAGE_BYTES = 2 * TILE_BYTES;  // A + B
-
 enum Mode { ROWCOL = 0, BLOCKWISE = 1 };
-// Epilogue staging: each wave's 128 x 128 bf16 result, rows padded to 272 B so
-// the 16-byte row reads of the store pass are conflict-free.
-constexpr int OUT_ROW = 128 * 2 + 16;
-constexpr int OUT_WAVE_BYTES = 128 * OUT_ROW;
-constexpr int SMEM_BYTES = (4 * OUT_WAVE_BYTES > 2 * STAGE_BYTES) ? 4 * OUT_WAVE_BYTES : 2 * STAGE_BYTES;
 constexpr int kMaxKT = 256;  // K <= 32768
 
 struct Params {
@@ -61,15 +58,12 @@ struct Params {
     // (the last row stripe if M % 256 != 0, then the last column stripe if
     // N % 256 != 0); each class is split evenly over the 8 XCDs.
     int tm_full, tn_full, tiles_full, tiles_part, m_tail;
-    // Tile width in columns: 256, except in the persistent row/column kernel,
-    // which takes 192 when a launch has fewer 256-wide tiles than CUs and
-    // more, still at most one per CU, at 192 (its WC template argument).
-    int bn;
     // Persistent kernel: rows [M, tail_M) (tail_M > M only when the tail
     // stripe rides on the light workgroups, tail_wide) in items of tail_cols
     // columns, item i for light workgroup i.
     int64_t tail_M;
     int tail_cols;
+    int group;  // gemm_small_kernel: tile rows per group of its work order
 };
 
 // 16-byte chunk c of LDS row r lives at chunk position c ^ ((r >> 1) & 7).
@@ -121,29 +115,6 @@ HN_DEVICE f32x16 mfma(const i32x8& a, const i32x8& b, const f32x16& c) {
     return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
 }
 
-// The eight fragments (4 weight blocks, 4 activation blocks) of one 64-byte
-// K slice of a stage, for the wave's 128 x 128 sub-tile.
-struct Frags {
-    i32x8 b[4];
-    i32x8 a[4];
-};
-
-HN_DEVICE void mfma_slice(f32x16 (&acc)[4][4], const Frags& f) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = mfma(f.b[i], f.a[j], acc[i][j]);
-}
-
-// Interleave the 16 LDS reads of the next slice with this slice's 16 MFMAs.
-HN_DEVICE void interleave_reads_with_mfma() {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one DS read
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-    }
-}
-
 HN_DEVICE float gelu_tanh(float x) {
     // 0.5 x (1 + tanh(u)) with u = sqrt(2/pi) (x + 0.044715 x^3), written as
     // x * sigmoid(2u) = x / (1 + 2^t), t = -2 u log2(e) = x (c0 + c1 x^2), on
@@ -162,117 +133,19 @@ HN_DEVICE uint32_t pack_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
 
-// Epilogue shared by the kernels. acc[i][j][v] holds out^T for n = wn*128 +
-// 32 i + 8 (v/4) + 4 (lane/32) + v%4 and m = wm*128 + 32 j + lane%32
-// (tile-local). Each wave scales its 128 x 128 sub-tile, packs it to bf16 and
-// parks it in its own LDS slice; then it writes the slice out as 256-byte row
-// segments (16 lanes x 16 bytes per row, 4 rows per store).
-//
-// The per-row / per-column scales and the bias the lane needs (4 + 16 x 4 +
-// 16 x 4 values) are loaded in one batch up front: with one wave per SIMD
-// nothing else hides a load's latency, so loading them group by group would
-// expose it sixteen times.
-template <int MODE, int ACT>
-HN_DEVICE void epilogue_act(f32x16 (&acc)[4][4], const Params& p, int64_t m0, int64_t n0, uint8_t* smem,
-                            int wave, int wm, int wn, int lane, int imax, int jmax) {
-    float sam[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        int64_t m = m0 + wm * 128 + j * 32 + (lane & 31);
-        m = m < p.M ? m : p.M - 1;
-        sam[j] = MODE == ROWCOL ? p.sa[m] : 1.0f;
-    }
-    float4 sbn[4][4];
-    uint2 bias[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int vq = 0; vq < 4; ++vq) {
-            int64_t n = n0 + wn * 128 + i * 32 + vq * 8 + (lane >> 5) * 4;
-            n = n < p.N ? n : p.N - 4;  // stays in bounds; columns past N are not stored
-            sbn[i][vq] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-            bias[i][vq] = make_uint2(0u, 0u);
-            if (MODE == ROWCOL) {
-                sbn[i][vq] = *reinterpret_cast<const float4*>(p.sb + n);
-                if (p.bias) bias[i][vq] = *reinterpret_cast<const uint2*>(p.bias + n);
-            }
-        }
-    __syncthreads();  // the last K step's LDS reads are done (all waves)
-    uint8_t* ow = smem + wave * OUT_WAVE_BYTES;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (i >= imax) continue;  // weight block wholly past N (wave-uniform)
-#pragma unroll
-        for (int vq = 0; vq < 4; ++vq) {
-            const float sb4[4] = {sbn[i][vq].x, sbn[i][vq].y, sbn[i][vq].z, sbn[i][vq].w};
-            const uint2 bb = bias[i][vq];
-            const float bn[4] = {bf16_bits_to_f32(bb.x & 0xffffu), bf16_bits_to_f32(bb.x >> 16),
-                                 bf16_bits_to_f32(bb.y & 0xffffu), bf16_bits_to_f32(bb.y >> 16)};
-            const int nl = i * 32 + vq * 8 + (lane >> 5) * 4;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (j >= jmax) continue;  // activation block wholly past M (wave-uniform)
-                float y[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    y[e] = fmaf(acc[i][j][vq * 4 + e], sam[j] * sb4[e], bn[e]);
-                    if (ACT == HN_ACT_GELU_TANH) y[e] = gelu_tanh(y[e]);
-                }
-                const int ml = j * 32 + (lane & 31);
-                *reinterpret_cast<uint2*>(ow + ml * OUT_ROW + nl * 2) =
-                    make_uint2(pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]));
-            }
-        }
-    }
-    // Each wave reads back only its own slice: no barrier needed beyond the
-    // wave's own LDS ordering.
-    __builtin_amdgcn_s_waitcnt(0);
-    const int64_t nbase = n0 + wn * 128 + (lane & 15) * 8;
-#pragma unroll 4
-    for (int r = 0; r < 32; ++r) {
-        const int ml = r * 4 + (lane >> 4);
-        const int64_t m = m0 + wm * 128 + ml;
-        const uint4 v = *reinterpret_cast<const uint4*>(ow + ml * OUT_ROW + (lane & 15) * 16);
-        if (m < p.M && nbase < p.N) *reinterpret_cast<uint4*>(p.out + m * p.ldc + nbase) = v;
-    }
-}
-
-template <int MODE>
-HN_DEVICE void epilogue(f32x16 (&acc)[4][4], const Params& p, int64_t m0, int64_t n0, uint8_t* smem,
-                        int wave, int wm, int wn, int lane, int imax = 4, int jmax = 4) {
-    if (MODE == ROWCOL && p.act == HN_ACT_GELU_TANH)
-        epilogue_act<MODE, HN_ACT_GELU_TANH>(acc, p, m0, n0, smem, wave, wm, wn, lane, imax, jmax);
-    else
-        epilogue_act<MODE, HN_ACT_NONE>(acc, p, m0, n0, smem, wave, wm, wn, lane, imax, jmax);
-}
-
 // ---------------------------------------------------------------------------
-// Row/column-scaled kernel: 128-byte K steps through five single-operand LDS
-// buffers.
+// K pipeline of the 256 x 256 tiles: 128-byte K steps through single-operand
+// LDS buffers.
 //
 // The stage DMA costs per cache line touched: one CU moves a 32 KB stage of
 // 128-byte row segments in about 810 cycles, but one of 64-byte segments (half
 // lines) in about 1360 -- more than the 1024 MFMA cycles a 64-byte K step of a
 // 256 x 256 tile takes. So every LDS buffer holds whole lines: one operand's
 // 256 rows x 128 bytes (32 KB, 16-byte chunks swizzled as swz()). Five buffers
-// fill the 160 KB of LDS; load L(i) -- A of K step i / 2 for even i, B for odd
-// i -- goes to buffer i % 5.
-//
-// K step k (128 bytes) runs as two halves of 16 MFMAs, one per 64-byte K slice,
-// each interleaved with the 16 LDS reads of the next slice's fragments:
-//   half 0: MFMAs on slice (k, 0); reads of slice (k, 1)
-//   mid:    wait for step k + 1's buffers and barrier; step k's buffers are
-//           then free (their last reads completed before the barrier)
-//   half 1: MFMAs on slice (k, 1); reads of slice (k + 1, 0); the loads
-//           L(2k + 5) = B(k + 2) and L(2k + 6) = A(k + 3) into step k's
-//           buffers, one 1 KB DMA per MFMA
-// B of a step is requested about one step (32 MFMAs) before its wait, A two
-// steps; with that lead the waits measure ~0 cycles per tile.
+// fill the 160 KB of LDS.
 constexpr int R_BUFS = 5;
 constexpr int R_BUF = BM * BK;            // one operand of one K step, 32 KB
 constexpr int R_SMEM = R_BUFS * R_BUF;    // 160 KB
-static_assert(R_SMEM >= 4 * OUT_WAVE_BYTES, "epilogue staging must fit in the stage buffers");
-
 // Stage loads use global_load_lds with a scalar base: the address is
 // sbase (SGPR pair: operand + tile row0 * K + k0) + voff (per-lane 32-bit
 // offset of the lane's row and chunk inside the tile, fixed for the tile), and
@@ -286,42 +159,6 @@ HN_DEVICE void dma_16B_sbase(const uint8_t* sbase, uint32_t voff, uint32_t lds) 
         : "v"(voff), "s"(sbase), "s"(lds)
         : "memory", "m0");
 }
-
-// Per-lane offsets of a wave's eight 1 KB regions (8 rows of 128 bytes) of one
-// 256 x 128 buffer. Lane l lands at row l / 8, physical chunk l % 8 of region
-// wave * 8 + q and fetches the logical chunk that position holds (the swizzle
-// is an involution). Rows past the operand's end are clamped to its last row:
-// in bounds, never stored.
-HN_DEVICE void buffer_offsets(uint32_t (&off)[8], int64_t row0, int64_t rows, int64_t K, int wave, int lane) {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        const int r = (wave * 8 + q) * 8 + (lane >> 3);
-        const int c = swz_pos(r, lane & 7);
-        const int64_t row = row0 + r < rows ? row0 + r : rows - 1;
-        off[q] = (uint32_t)((row - row0) * K + (c << 4));
-    }
-}
-
-// The fragments of K slice kh of step buffers (a_buf, b_buf).
-HN_DEVICE void read_slice(Frags& f, const uint8_t* a_buf, const uint8_t* b_buf, int kh, int wm, int wn,
-                          int lane) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) f.b[i] = read_frag(b_buf, wn * 128 + i * 32 + (lane & 31), kh, lane);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) f.a[j] = read_frag(a_buf, wm * 128 + j * 32 + (lane & 31), kh, lane);
-}
-
-// mfma_slice for an edge tile: only blocks inside the matrix (wave-uniform tests).
-HN_DEVICE void mfma_slice_partial(f32x16 (&acc)[4][4], const Frags& f, int imax, int jmax) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (i < imax && j < jmax) acc[i][j] = mfma(f.b[i], f.a[j], acc[i][j]);
-}
-
-// One workgroup per queue entry (id = x + 8 i).
-HN_DEVICE bool tile_of(const Params& p, int id, int& tm, int& tn) { return tile_at(p, id & 7, id >> 3, tm, tn); }
 
 // ---------------------------------------------------------------------------
 // Blockwise-scaled kernel, 8 waves: a 512-thread workgroup owns a 256 x 256
@@ -550,160 +387,6 @@ __global__ __launch_bounds__(NT8, 1) void gemm_bw8_kernel(Params p) {
         }
 }
 
-__global__ __launch_bounds__(NT, 1) void gemm_rowcol_kernel(Params p) {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[R_SMEM];
-    int tm, tn;
-    if (!tile_of(p, blockIdx.x, tm, tn)) return;
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
-    const int KT = (int)(p.K / BK);
-    const uint8_t* const a_tile = p.a + m0 * p.K;
-    const uint8_t* const b_tile = p.b + n0 * p.K;
-    uint32_t off_a[8], off_b[8];
-    buffer_offsets(off_a, m0, p.M, p.K, wave, lane);
-    buffer_offsets(off_b, n0, p.N, p.K, wave, lane);
-    const uint32_t lds_base = lds_addr(smem) + wave * 8 * 1024;
-    // Blocks of this wave inside the matrix: imax weight blocks (N % 128 == 0,
-    // so 0 or 4), jmax activation blocks of 32 rows. Wave-uniform.
-    const int64_t rows_w = p.M - (m0 + wm * 128), cols_w = p.N - (n0 + wn * 128);
-    const int jmax = rows_w >= 128 ? 4 : (rows_w <= 0 ? 0 : (int)((rows_w + 31) >> 5));
-    const int imax = cols_w >= 128 ? 4 : (cols_w <= 0 ? 0 : (int)(cols_w >> 5));
-    const bool whole = imax == 4 && jmax == 4;
-
-    f32x16 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-    // Buffers of step s: A in (2 s) % 5, B in (2 s + 1) % 5.
-    auto a_buf = [&](int s) { return smem + ((2 * s) % R_BUFS) * R_BUF; };
-    auto b_buf = [&](int s) { return smem + ((2 * s + 1) % R_BUFS) * R_BUF; };
-    auto issue_a = [&](int s) {
-        const uint32_t dst = lds_base + ((2 * s) % R_BUFS) * R_BUF;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) dma_16B_sbase(a_tile + (int64_t)s * BK, off_a[q], dst + q * 1024);
-    };
-    auto issue_b = [&](int s) {
-        const uint32_t dst = lds_base + ((2 * s + 1) % R_BUFS) * R_BUF;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) dma_16B_sbase(b_tile + (int64_t)s * BK, off_b[q], dst + q * 1024);
-    };
-    // Prologue: L(0) .. L(4), then wait for step 0 (L(0), L(1)).
-    issue_a(0);
-    issue_b(0);
-    if (KT > 1) {
-        issue_a(1);
-        issue_b(1);
-        if (KT > 2) {
-            issue_a(2);
-            asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        }
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    __syncthreads();
-
-    // The K loop, instantiated for whole tiles and for edge tiles (blocks
-    // outside the matrix skipped); the choice is made once per tile.
-    auto kloop = [&](auto edge_tag) {
-        constexpr bool EDGE = decltype(edge_tag)::value;
-        Frags cur, nxt;
-        auto mfmas = [&](const Frags& f) {
-            if (EDGE) {
-                mfma_slice_partial(acc, f, imax, jmax);
-            } else {
-                mfma_slice(acc, f);
-                interleave_reads_with_mfma();
-            }
-        };
-        // half 0 of step k: MFMAs on slice (k, 0), reads of slice (k, 1)
-        auto half0 = [&](int k) {
-            read_slice(nxt, a_buf(k), b_buf(k), 1, wm, wn, lane);
-            mfmas(cur);
-        };
-        // half 1 of step k: MFMAs on slice (k, 1), reads of slice (k + 1, 0)
-        auto half1 = [&](int k) {
-            read_slice(cur, a_buf(k + 1), b_buf(k + 1), 0, wm, wn, lane);
-            mfmas(nxt);
-        };
-        read_slice(cur, a_buf(0), b_buf(0), 0, wm, wn, lane);
-        int k = 0;
-        // Steady state: at the mid-step wait, A(k + 2) is still in flight.
-        // Half 1 of a steady-state step with the step's 16 DMA issues spread
-        // one per MFMA: a DMA issue stalls the wave while the address unit
-        // takes its 1 KB, and back to back after the barrier the 16 of them
-        // kept the matrix core idle for about 1000 cycles per step. Slot s
-        // holds one fragment read of slice (k + 1, 0) (s < 8), MFMA s on slice
-        // (k, 1) and DMA s (B(k + 2) regions, then A(k + 3) regions); the
-        // sched_barrier keeps each slot's instructions together.
-        auto half1_dma = [&](int k, auto with_a_tag) {
-            constexpr bool WITH_A = decltype(with_a_tag)::value;
-            const uint8_t* an = a_buf(k + 1);
-            const uint8_t* bn = b_buf(k + 1);
-            const uint32_t db = lds_base + ((2 * (k + 2) + 1) % R_BUFS) * R_BUF;
-            const uint32_t da = lds_base + ((2 * (k + 3)) % R_BUFS) * R_BUF;
-            const uint8_t* bsrc = b_tile + (int64_t)(k + 2) * BK;
-            const uint8_t* asrc = a_tile + (int64_t)(k + 3) * BK;
-#pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                if (s < 4) cur.b[s] = read_frag(bn, wn * 128 + s * 32 + (lane & 31), 0, lane);
-                else if (s < 8) cur.a[s - 4] = read_frag(an, wm * 128 + (s - 4) * 32 + (lane & 31), 0, lane);
-                acc[s >> 2][s & 3] = mfma(nxt.b[s >> 2], nxt.a[s & 3], acc[s >> 2][s & 3]);
-                if (s < 8) dma_16B_sbase(bsrc, off_b[s], db + s * 1024);
-                else if (WITH_A) dma_16B_sbase(asrc, off_a[s - 8], da + (s - 8) * 1024);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-        if constexpr (!EDGE) {
-            for (; k + 3 < KT; ++k) {
-                half0(k);
-                asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // step k + 1 landed (this wave)
-                __syncthreads();                                  // ... every wave; step k's buffers free
-                half1_dma(k, std::true_type{});
-            }
-            if (k + 2 < KT) {
-                half0(k);
-                asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-                __syncthreads();
-                half1_dma(k, std::false_type{});
-                ++k;
-            }
-        } else {
-            for (; k + 2 < KT; ++k) {
-                half0(k);
-                asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // step k + 1 landed (this wave)
-                __syncthreads();                                  // ... every wave; step k's buffers free
-                issue_b(k + 2);
-                if (k + 3 < KT) issue_a(k + 3);
-                half1(k);
-            }
-        }
-        if (k + 1 < KT) {  // k = KT - 2: nothing left to issue
-            half0(k);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            half1(k);
-            ++k;
-        }
-        // k = KT - 1: the last slice's MFMAs read nothing further.
-        read_slice(nxt, a_buf(k), b_buf(k), 1, wm, wn, lane);
-        mfmas(cur);
-        if (EDGE) mfma_slice_partial(acc, nxt, imax, jmax);
-        else mfma_slice(acc, nxt);
-    };
-    if (whole) kloop(std::false_type{});
-    else kloop(std::true_type{});
-    epilogue<ROWCOL>(acc, p, m0, n0, smem, wave, wm, wn, lane, imax, jmax);
-}
-
 // ===========================================================================
 // Overlapped-epilogue row/column kernel (K >= O_MIN_KT x 128): persistent,
 // one workgroup per CU walking its XCD's tile queue (tile_of order).
@@ -743,6 +426,7 @@ constexpr int O_BIAS_F32 = 1280;                    // the bias as fp32 (bias_to
 constexpr int O_STAGE_BASE = O_BUFS * R_BUF;
 constexpr int O_PARAM_BASE = O_STAGE_BASE + 4 * O_STAGE;
 constexpr int O_SMEM = O_PARAM_BASE + 4 * O_PARAMS;
+constexpr int O_WC = 128;                           // columns per wave
 constexpr int O_JO = 2;                             // row blocks carried into the next tile
 constexpr int O_PASSES = 2 * O_JO;                  // overlapped passes (steps 0 .. O_PASSES - 1)
 constexpr int O_MIN_KT = O_PASSES + 3;              // + the tail step + the last two steps
@@ -787,18 +471,17 @@ HN_DEVICE void dma_4B_sbase(const void* sbase, uint32_t voff, uint32_t lds) {
 // are clamped to the operand's end (in bounds; never used). bias_to_f32 then
 // widens the bias to fp32 at [1280, 1792), so the epilogue reads 4 biases as
 // one 16-byte load with no per-value conversion.
-template <int WC>
 HN_DEVICE void param_dma(const Params& p, int64_t m0, int64_t n0, int wm, int wn, int lane, uint32_t lds, int q) {
     if (q < 2) {
         int64_t m = m0 + wm * 128 + 64 * q + lane;
         m = m < p.M ? m : p.M - 1;
         dma_4B_sbase(p.sa, (uint32_t)(m * 4), lds + 256 * q);
     } else if (q < 4) {
-        int64_t n = n0 + wn * WC + 64 * (q - 2) + lane;
+        int64_t n = n0 + wn * O_WC + 64 * (q - 2) + lane;
         n = n < p.N ? n : p.N - 1;
         dma_4B_sbase(p.sb, (uint32_t)(n * 4), lds + 512 + 256 * (q - 2));
     } else if (p.bias) {
-        int64_t n = n0 + wn * WC + 2 * lane;
+        int64_t n = n0 + wn * O_WC + 2 * lane;
         n = n < p.N ? n : p.N - 2;
         dma_4B_sbase(p.bias, (uint32_t)(n * 2), lds + 1024);
     } else {
@@ -893,17 +576,16 @@ HN_DEVICE uint4 oe_readback(const uint8_t* stg, int q, int lane) {
 
 // Store q of pass P of the pending sub-tile (gemm_dma.h: oe_store_off), through
 // its output window (pimax: its column blocks inside the matrix).
-template <int WC>
 HN_DEVICE void oe_store(__amdgpu_buffer_rsrc_t win, int pimax, uint32_t pitch, int P, int q, const uint4& v,
                         int lane) {
-    if (oe_store_on(WC, pimax, P, lane))
+    if (oe_store_on(O_WC, pimax, P, lane))
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), win,
                                                (int)oe_store_off(pitch, lane, P, q), 0, 0);
 }
 
 // All eight passes of a pending tile without overlap (before an edge tile and
 // after a workgroup's last tile).
-template <int ACT, int WC>
+template <int ACT>
 HN_DEVICE void oe_flush(const Params& p, uint32_t (&y)[4][4][8], uint8_t* stg, __amdgpu_buffer_rsrc_t win,
                         int pimax, int lane) {
     const uint32_t pitch = (uint32_t)p.ldc * 2;
@@ -915,7 +597,7 @@ HN_DEVICE void oe_flush(const Params& p, uint32_t (&y)[4][4][8], uint8_t* stg, _
 #pragma unroll
         for (int g = 0; g < 4; ++g) oe_write(y, stg, P, g >> 1, g & 1, lane);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) oe_store<WC>(win, pimax, pitch, P, q, oe_readback(stg, q, lane), lane);
+        for (int q = 0; q < 4; ++q) oe_store(win, pimax, pitch, P, q, oe_readback(stg, q, lane), lane);
     }
 }
 
@@ -926,7 +608,7 @@ HN_DEVICE void oe_flush(const Params& p, uint32_t (&y)[4][4][8], uint8_t* stg, _
 // LDS staging of the carried passes: a store writes 32 bytes of each of 32
 // rows (the two half waves side by side), and the 4 stores of a pass fill its
 // rows' 128-byte lines, which the L2 merges.
-template <int ACT, int WC>
+template <int ACT>
 HN_DEVICE void direct_passes(const Params& p, const f32x16 (&acc)[4][4], const uint8_t* prm,
                              __amdgpu_buffer_rsrc_t win, int imax, int lane) {
     const int h = lane >> 5, r = oe_row(lane & 31);
@@ -945,7 +627,6 @@ HN_DEVICE void direct_passes(const Params& p, const f32x16 (&acc)[4][4], const u
 #pragma unroll
         for (int ii = 0; ii < 2; ++ii) {
             const int i = 2 * ih + ii;
-            if (32 * i >= WC) continue;  // block past a 96-column wave
             uint32_t w[8];
 #pragma unroll
             for (int vq = 0; vq < 4; ++vq) {
@@ -968,7 +649,7 @@ HN_DEVICE void direct_passes(const Params& p, const f32x16 (&acc)[4][4], const u
                 w[2 * vq] = o.x;
                 w[2 * vq + 1] = o.y;
             }
-            if (direct_store_on(WC, imax, i)) {
+            if (direct_store_on(O_WC, imax, i)) {
                 __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{w[0], w[1], w[2], w[3]}, win,
                                                        (int)direct_store_off(pitch, lane, P, ii, 0), 0, 0);
                 __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{w[4], w[5], w[6], w[7]}, win,
@@ -1107,11 +788,9 @@ HN_DEVICE void tail_wide(const Params& p, int64_t m0, int64_t M, int64_t n0, int
     }
 }
 
-// WC: columns per wave, 128 (256 x 256 tiles) or 96 (256 x 192 tiles, which
-// take the edge-tile path: no carried epilogue).
-template <int ACT, int WC>
+template <int ACT>
 __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
-    constexpr int TBN = 2 * WC;  // tile columns
+    constexpr int TBN = 2 * O_WC;  // tile columns
     __shared__ __attribute__((aligned(16))) uint8_t smem[O_SMEM];
     const int xcd = blockIdx.x & 7;
     const int stride = (int)(gridDim.x >> 3);  // workgroups per XCD
@@ -1119,7 +798,6 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
     int tm, tn;
     if (!tile_of_slot(p, xcd, slot, stride, tm, tn)) return;
 
-    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave & 1, wn = wave >> 1;
     const int KT = (int)(p.K / BK);
@@ -1145,8 +823,6 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
         a_src = p.a + m0_ * p.K;
         b_src = p.b + n0_ * p.K;
         const int64_t a_rows = p.M - m0_ < BM ? p.M - m0_ : BM;
-        // A 192-wide tile still fills all 256 stage rows; rows past its width
-        // are clamped like rows past N (never read by an MFMA).
         const int64_t b_rows = p.N - n0_ < TBN ? p.N - n0_ : TBN;
         a_lim = dma_limit(a_rows, p.K);
         b_lim = dma_limit(b_rows, p.K);
@@ -1167,7 +843,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
     auto set_cur = [&](int tm_, int tn_) {
         cm0 = (int64_t)tm_ * BM;
         cn0 = (int64_t)tn_ * TBN;
-        const WaveExtent e = wave_extent(p.M, p.N, cm0 + wm * 128, cn0 + wn * WC, WC);
+        const WaveExtent e = wave_extent(p.M, p.N, cm0 + wm * 128, cn0 + wn * O_WC, O_WC);
         cimax = e.imax;
         cjmax = e.jmax;
     };
@@ -1220,13 +896,13 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
         fa[j] = frag_at(buf, wm * 128 + j * 32, kh, d);
     };
     auto read_b = [&](const uint8_t* buf, int i, int kh, const RdLane& d) {
-        fb[i] = frag_at(buf, wn * WC + i * 32, kh, d);
+        fb[i] = frag_at(buf, wn * O_WC + i * 32, kh, d);
     };
     // Rolling reads of the next slice after slot s's MFMA.
     auto roll = [&](int s, const uint8_t* abuf, const uint8_t* bbuf, int kh, const RdLane& d) {
         if (s == 3 || s == 7 || s == 11) read_b(bbuf, s >> 2, kh, d);
         if (s >= 12) read_a(abuf, s - 12, kh, d);
-        if (s == 15 && WC == 128) read_b(bbuf, 3, kh, d);  // no fourth block at 96 columns
+        if (s == 15) read_b(bbuf, 3, kh, d);
     };
 
     // One K step. EDGE: edge tile (blocks outside the matrix skipped). PASS:
@@ -1257,7 +933,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
 #pragma unroll
         for (int s = 0; s < 16; ++s) {
             const int i = s >> 2, j = s & 3;
-            if (i < WC / 32 && (!EDGE || (i < cimax && j < cjmax))) {
+            if (!EDGE || (i < cimax && j < cjmax)) {
                 if (FIRST) acc[i][j] = mfma(fb[i], fa[j], f32x16{});
                 else acc[i][j] = mfma(fb[i], fa[j], acc[i][j]);
             } else if (FIRST) {
@@ -1277,9 +953,9 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
             // staging writes (slots 3-15), stores two slots after each read.
             if (PASS >= 1 && s < 4) rb[s] = oe_readback(stg, s, el);
             if (PASS >= 1 && s >= 2 && s < 6)
-                oe_store<WC>(pwin, pimax, pitch, PASS - 1, s - 2, rb[s - 2], el);
+                oe_store(pwin, pimax, pitch, PASS - 1, s - 2, rb[s - 2], el);
             const int i = s >> 2, j = s & 3;
-            if (i < WC / 32 && (!EDGE || (i < cimax && j < cjmax))) acc[i][j] = mfma(fb[i], fa[j], acc[i][j]);
+            if (!EDGE || (i < cimax && j < cjmax)) acc[i][j] = mfma(fb[i], fa[j], acc[i][j]);
             if (NEXT) roll(s, an, bnx, 0, rl);
             if (DMA == 1 || DMA == 3) {
                 if (s < 8) dma_a(dl, k + 2, dst, s);
@@ -1289,7 +965,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
                 if (s < 8) dma_a(dl, 0, dst, s);
                 else dma_b(dl, 0, dst, s - 8);
             }
-            if (DMA == 3 && s >= 8 && s < 13) param_dma<WC>(p, cm0, cn0, wm, wn, el, prm_lds, s - 8);
+            if (DMA == 3 && s >= 8 && s < 13) param_dma(p, cm0, cn0, wm, wn, el, prm_lds, s - 8);
             if (DMA == 0 && !NEXT && s == 2) bias_to_f32(prm, el);  // the last step: its slots are free
             if (PASS >= 0 && PASS < O_PASSES) {
                 oe_act<ACT>(y, glo, PASS, 16 + s);
@@ -1338,11 +1014,11 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
             const RdLane d = rd_lane(fresh_lane());
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                if (q < WC / 32) read_b(ab + R_BUF, q, 0, d);
+                read_b(ab + R_BUF, q, 0, d);
                 read_a(ab, q, 0, d);
             }
         }
-        const bool whole = cimax == WC / 32 && cjmax == 4;
+        const bool whole = cimax == 4 && cjmax == 4;
         if (whole) {
             if (!pending) {
                 // Nothing carried yet: the passes run on zeros, their stores
@@ -1368,7 +1044,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
             step(KT - 1, F{}, std::integral_constant<int, -1>{}, std::integral_constant<int, 0>{}, F{}, F{});
             stamp(2);
         } else {
-            if (pending) oe_flush<ACT, WC>(p, y, stg, pwin, pimax, fresh_lane());
+            if (pending) oe_flush<ACT>(p, y, stg, pwin, pimax, fresh_lane());
             step(0, T{}, std::integral_constant<int, -1>{}, std::integral_constant<int, 3>{}, T{}, T{});
             for (int k = 1; k < KT - 2; ++k)
                 step(k, T{}, std::integral_constant<int, -1>{}, std::integral_constant<int, 1>{}, T{}, F{});
@@ -1389,8 +1065,8 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
             for (int q = 0; q < 8; ++q) dma_b(d, 1, pr, q);
         }
         stamp(4);
-        const __amdgpu_buffer_rsrc_t cwin = out_window(p, cm0 + wm * 128, cn0 + wn * WC, cimax);
-        direct_passes<ACT, WC>(p, acc, prm, cwin, cimax, fresh_lane());
+        const __amdgpu_buffer_rsrc_t cwin = out_window(p, cm0 + wm * 128, cn0 + wn * O_WC, cimax);
+        direct_passes<ACT>(p, acc, prm, cwin, cimax, fresh_lane());
         stamp(5);
         convert_tile(acc, y, prm, fresh_lane());
         stamp(6);
@@ -1409,7 +1085,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
         ++stamp_tile;
 #endif
     }
-    oe_flush<ACT, WC>(p, y, stg, pwin, pimax, fresh_lane());
+    oe_flush<ACT>(p, y, stg, pwin, pimax, fresh_lane());
     // The last step's re-load of step 0 (no next tile) may still be landing.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (p.tail_M > p.M) {
@@ -1606,10 +1282,438 @@ __global__ __launch_bounds__(64 * SK) void gemm_tail_kernel(Params p, int64_t m0
     }
 }
 
+// ---------------------------------------------------------------------------
+// Launches that 256 x 256 tiles would leave uneven or mostly idle (a text
+// stream's linears, a short batch, 9 rounds for 8.1 rounds of work), and short
+// K: tiles of 32 WR RB rows x 32 WC CB columns.
+//
+// A workgroup of WR x WC waves owns one tile, each wave RB x CB MFMA blocks. A K
+// step (128 bytes of every row of both operands) is one LDS stage of whole
+// 128-byte lines, filled by all waves' direct loads in the persistent kernel's
+// swizzled layout; S of them are in flight. Step t's MFMAs run from registers
+// beside the LDS reads of the next fragments and the loads of step t + S into
+// step t's stage, one barrier a step. The fragment rows follow oe_row, so a lane
+// stores 8 consecutive columns (16 bytes). ROWCOL sums each output by the
+// persistent kernel's own MFMA chain (bit-identical to it).
+//
+// What bounds it: up to about 64 tiles, the loads' rate into one CU (about 45
+// bytes a cycle: a step costs by its rows); with a tile on every CU, the L2s'
+// (11-15 TB/s in all), so larger tiles and the group order (small_tile; 10800 x
+// 3072 -> 12288 in 256 x 192 tiles 432 -> 365 us with it) matter there. Measured
+// against the 256 x 256 tiles (GEMM alone): 256 x 12288 -> 3072 95 -> 22 us,
+// 256 x 3072 -> 9216 31 -> 16 us, 4096 x 3072 -> 9216 118 -> 103 us, 4000 x 512
+// -> 1536 17.0 -> 9.7 us; blockwise 1536 x 12288 -> 4096 127 -> 87 us, 256 x
+// 4096 -> 4096 47 -> 13 us.
+constexpr int small_stage_bytes(int tm, int tn) { return (tm + tn) * BK; }
+constexpr int small_stages(int tm, int tn) {
+    return R_SMEM / small_stage_bytes(tm, tn) < 5 ? R_SMEM / small_stage_bytes(tm, tn) : 5;
+}
+
+template <int MODE, int ACT, int WR, int WC, int RB, int CB>
+__global__ __launch_bounds__(64 * WR * WC, MODE == BLOCKWISE || WR * WC == 8 ? 2 : 1) void gemm_small_kernel(
+    Params p, int round_first) {
+    constexpr int TM = 32 * WR * RB, TN = 32 * WC * CB, STG = small_stage_bytes(TM, TN), S = small_stages(TM, TN);
+    constexpr int NQ = (TM + TN) / (8 * WR * WC);  // 1 KB loads per wave and step
+    static_assert(NQ * 8 * WR * WC == TM + TN && 4 * NQ < 64 && S >= 2, "whole loads per wave");
+    // Fragment buffering: two whole steps, or, where that takes too many
+    // registers, two K slices.
+    constexpr bool SLICED = MODE == BLOCKWISE ? RB * CB >= 4 : RB * CB >= (WR * WC == 8 ? 3 : 8);
+    // Dynamic, S * STG bytes: with its size in sight the compiler takes one
+    // wave per SIMD for granted and moves BLOCKWISE's accumulators to AGPRs.
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    // Workgroup ids go round-robin to the XCDs: an XCD takes consecutive work
+    // items, in groups of p.group tile rows walking N, so the tiles it runs at
+    // once share their A and B panels in its L2.
+    const int item = (int)(blockIdx.x & 7) * p.per_xcd + (int)(blockIdx.x >> 3);
+    if (item >= p.tiles_m * p.tiles_n) return;
+    int tm, tn;
+    small_tile(item, p.tiles_m, p.tiles_n, p.group, tm, tn);
+    const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = w % WR, wc = w / WR;
+    const int64_t K = p.K;
+    const int KT = (int)(K / BK);
+    const uint32_t lds0 = lds_addr(smem) + w * NQ * 1024;
+
+    const uint8_t* src[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const TailSrc ts = tail_wide_src(w * NQ + q, lane, TM, m0, p.M, n0, p.N - 1, K);
+        src[q] = (ts.a ? p.a : p.b) + ts.off;
+    }
+    const int64_t mw = m0 + wr * 32 * RB, nw = n0 + wc * 32 * CB;  // the wave's blocks
+    const int rl = oe_row(lane & 31);
+    // This lane's scales and bias: loaded ahead of the K loop's direct loads,
+    // or behind it where the K loop needs the registers.
+    constexpr bool EARLY = RB + CB <= 4 && WR * WC == 4;
+    float sam[RB], sbv[CB][2][8];
+    uint4 bias[CB][2];
+    auto load_scales = [&]() {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            const int64_t m = mw + 32 * r + rl;
+            sam[r] = p.sa[m < p.M ? m : p.M - 1];
+        }
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                int64_t n = nw + 32 * c + 16 * h + 8 * (lane >> 5);
+                n = n < p.N ? n : p.N - 8;  // in bounds; columns past N are not stored
+                const float4 s0 = *reinterpret_cast<const float4*>(p.sb + n);
+                const float4 s1 = *reinterpret_cast<const float4*>(p.sb + n + 4);
+                sbv[c][h][0] = s0.x; sbv[c][h][1] = s0.y; sbv[c][h][2] = s0.z; sbv[c][h][3] = s0.w;
+                sbv[c][h][4] = s1.x; sbv[c][h][5] = s1.y; sbv[c][h][6] = s1.z; sbv[c][h][7] = s1.w;
+                bias[c][h] = make_uint4(0u, 0u, 0u, 0u);
+                if (p.bias) {
+                    const uint2 b0 = *reinterpret_cast<const uint2*>(p.bias + n);
+                    const uint2 b1 = *reinterpret_cast<const uint2*>(p.bias + n + 4);
+                    bias[c][h] = make_uint4(b0.x, b0.y, b1.x, b1.y);
+                }
+            }
+    };
+    if (MODE == ROWCOL && EARLY) load_scales();
+    // BLOCKWISE: the wave's blocks lie in one 128 x 128 scale block, so a step
+    // has one factor. The scale rows are read through the constant address
+    // space (scalar loads, outside the vector-memory counter that the stage
+    // waits count).
+    static_assert(MODE == ROWCOL || (128 % (32 * RB) == 0 && 128 % (32 * CB) == 0), "one factor per wave and step");
+    typedef const __attribute__((address_space(4))) float cfloat;
+    cfloat* sa_row = nullptr;
+    cfloat* sb_row = nullptr;
+    if (MODE == BLOCKWISE) {
+        sa_row = (cfloat*)p.sa + ((mw < p.M ? mw : p.M - 1) >> 7) * KT;
+        sb_row = (cfloat*)p.sb + ((nw < p.N ? nw : p.N - 1) >> 7) * KT;
+    }
+
+    auto issue = [&](int t, int q) {
+        dma_16B(src[q] + (int64_t)t * BK, lds0 + (t % S) * STG + q * 1024);
+    };
+    // Fragment t of a step: CB weight blocks, then RB activation blocks, of
+    // K slice t / (RB + CB).
+    constexpr int NF = RB + CB;
+    struct Step {
+        i32x8 f[2 * NF];
+    };
+    uint32_t foff[2][2];  // [K slice][chunk half], from the block's first row
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+        for (int hi = 0; hi < 2; ++hi)
+            foff[kh][hi] = (uint32_t)(rl * BK + (swz_pos(rl, 4 * kh + 2 * (lane >> 5) + hi) << 4));
+    auto read = [&](i32x8& f, int t, int i) {
+        const int kh = i / NF, b = i % NF;
+        const int row = b < CB ? TM + wc * 32 * CB + 32 * b : wr * 32 * RB + 32 * (b - CB);
+        const uint8_t* const at = smem + (t % S) * STG + row * BK;
+        const uint4 lo = *reinterpret_cast<const uint4*>(at + foff[kh][0]);
+        const uint4 hi = *reinterpret_cast<const uint4*>(at + foff[kh][1]);
+        f[0] = lo.x; f[1] = lo.y; f[2] = lo.z; f[3] = lo.w;
+        f[4] = hi.x; f[5] = hi.y; f[6] = hi.z; f[7] = hi.w;
+    };
+
+    f32x16 acc[RB][CB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int c = 0; c < CB; ++c) acc[r][c] = f32x16{};
+
+    const int first = KT < S ? KT : S;
+    for (int t = 0; t < first; ++t)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) issue(t, q);
+    // Waits until at most `left` steps' loads of this wave are in flight.
+    auto wait_steps = [&](int left) {
+        if (left >= 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * NQ) : "memory");
+        else if (left == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NQ) : "memory");
+        else if (left == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NQ) : "memory");
+        else if (left == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NQ) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    wait_steps(first - 1);
+    __syncthreads();
+    float f_out = 1.0f;  // BLOCKWISE: what the accumulators are in units of
+    if constexpr (SLICED) {
+        // The fragments double-buffer one K slice. BLOCKWISE, as
+        // gemm_bw8_kernel: the accumulators are kept in units of the current
+        // K block's factor (rescaled by f_prev / f before the block's first
+        // MFMA of the step), so that everything fits 256 VGPRs; a step whose
+        // factor is 0 has its fragments zeroed and the rescale 1.
+        constexpr int NB = RB * CB;
+        float f = 0.0f, q = 1.0f, f_next = 0.0f;  // step t's factor and rescale, step t + 1's factor
+        f_out = 0.0f;
+        if (MODE == BLOCKWISE) {
+            f = sa_row[0] * sb_row[0];
+            q = f != 0.0f ? f_out / f : 1.0f;
+        }
+        i32x8 f0[NF], f1[NF];  // slices 0 and 1
+#pragma unroll
+        for (int i = 0; i < NF; ++i) read(f0[i], 0, i);
+        auto step = [&](int t, auto more_t, auto load_t) {
+            constexpr bool MORE = decltype(more_t)::value, LOAD = decltype(load_t)::value;
+            constexpr int RPS = (NF + NB - 1) / NB, QPS = (NQ + NB - 1) / NB;  // reads, loads a slot
+            if (MODE == BLOCKWISE && MORE) f_next = sa_row[t + 1] * sb_row[t + 1];
+            if (MODE == BLOCKWISE && f == 0.0f)
+#pragma unroll
+                for (int i = 0; i < NF; ++i) f0[i] = i32x8{};
+            // Slice 0 beside the reads of slice 1.
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int r = i / CB, c = i % CB;
+#pragma unroll
+                for (int j = i * RPS; j < i * RPS + RPS; ++j)
+                    if (j < NF) read(f1[j], t, NF + j);
+                if (MODE == BLOCKWISE)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[r][c][v] *= q;
+                acc[r][c] = mfma(f0[c], f0[CB + r], acc[r][c]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (MODE == BLOCKWISE && f == 0.0f)
+#pragma unroll
+                for (int i = 0; i < NF; ++i) f1[i] = i32x8{};
+            if (MORE) {
+                // Step t's reads are done in this wave and step t + 1's loads have
+                // landed; past the barrier both hold for every wave, and step
+                // t's stage can be refilled.
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (LOAD) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * NQ) : "memory");
+                else wait_steps(KT - 2 - t);
+                __syncthreads();
+            }
+            // Slice 1 beside the reads of step t + 1's slice 0 and the loads of
+            // step t + S.
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int r = i / CB, c = i % CB;
+                acc[r][c] = mfma(f1[c], f1[CB + r], acc[r][c]);
+#pragma unroll
+                for (int j = i * RPS; j < i * RPS + RPS; ++j)
+                    if (MORE && j < NF) read(f0[j], t + 1, j);
+#pragma unroll
+                for (int j = i * QPS; j < i * QPS + QPS; ++j)
+                    if (LOAD && j < NQ) issue(t + S, j);
+                if (MODE == BLOCKWISE && MORE && i == 0) {
+                    if (f != 0.0f) f_out = f;
+                    f = f_next;
+                    q = f != 0.0f ? f_out / f : 1.0f;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!MORE && f != 0.0f) f_out = f;
+        };
+        int t = 0;
+        for (; t + S < KT; ++t) step(t, std::true_type{}, std::true_type{});
+        for (; t + 1 < KT; ++t) step(t, std::true_type{}, std::false_type{});
+        step(t, std::false_type{}, std::false_type{});
+    } else {
+    Step cur, nxt;
+#pragma unroll
+    for (int i = 0; i < 2 * NF; ++i) read(cur.f[i], 0, i);
+
+    // Step t from the fragments in c; n receives step t + 1's. MORE: a step
+    // t + 1 exists; LOAD: a step t + S exists.
+    constexpr int NM = 2 * RB * CB, SLOTS = NM > 2 * NF ? NM : 2 * NF;
+    auto step = [&](Step& c, Step& n, int t, auto more_t, auto load_t) {
+        constexpr bool MORE = decltype(more_t)::value, LOAD = decltype(load_t)::value;
+        if (MORE) {
+            // Step t's fragment reads are done in this wave (c is in registers)
+            // and step t + 1's loads have landed; past the barrier both hold
+            // for every wave, and step t's stage can be refilled.
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (LOAD) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * NQ) : "memory");
+            else wait_steps(KT - 2 - t);
+            __syncthreads();
+        }
+        // BLOCKWISE runs a block's two slices back to back and adds the block's
+        // product beside the next block's MFMAs.
+        f32x16 blk[2];
+        const float f = MODE == BLOCKWISE ? sa_row[t] * sb_row[t] : 1.0f;
+        auto promote = [&](int i) {
+            if (f != 0.0f) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    acc[i / CB][i % CB][v] = fmaf(blk[i & 1][v], f, acc[i / CB][i % CB][v]);
+            }
+        };
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s) {
+            if (s < NM) {
+                const int kh = MODE == ROWCOL ? s / (RB * CB) : s & 1, i = MODE == ROWCOL ? s % (RB * CB) : s >> 1;
+                const int r = i / CB, cc = i % CB;
+                const i32x8 &b = c.f[kh * NF + cc], &a = c.f[kh * NF + CB + r];
+                if (MODE == ROWCOL) acc[r][cc] = mfma(b, a, acc[r][cc]);
+                else blk[i & 1] = mfma(b, a, kh ? blk[i & 1] : f32x16{});
+            }
+            if (MORE && s < 2 * NF) read(n.f[s], t + 1, s);
+            if (LOAD && s < NQ) issue(t + S, s);
+            if (MODE == BLOCKWISE && s < NM && (s & 1) && s > 1) promote((s >> 1) - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (MODE == BLOCKWISE) promote(RB * CB - 1);
+    };
+    static_assert(SLOTS >= NQ, "every load has a slot");
+    using T = std::true_type;
+    using F = std::false_type;
+    int t = 0;
+    for (; t + S + 1 < KT; t += 2) {
+        step(cur, nxt, t, T{}, T{});
+        step(nxt, cur, t + 1, T{}, T{});
+    }
+    bool odd = false;  // the fragments of step t are in nxt
+    if (t + S < KT) {
+        step(cur, nxt, t++, T{}, T{});
+        odd = true;
+    }
+    for (; t + 1 < KT; ++t) {
+        if (odd) step(nxt, cur, t, T{}, F{});
+        else step(cur, nxt, t, T{}, F{});
+        odd = !odd;
+    }
+    if (odd) step(nxt, cur, t, F{}, F{});
+    else step(cur, nxt, t, F{}, F{});
+    }
+
+    if (MODE == ROWCOL && !EARLY) load_scales();
+    // acc[r][c][v] of lane l is output row oe_row(l % 32) of block r and column
+    // 16 (v / 8) + 8 (l / 32) + v % 8 of block c.
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        const int64_t m = mw + 32 * r + rl;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int64_t n = nw + 32 * c + 16 * h + 8 * (lane >> 5);
+                if (n >= p.N) continue;
+                uint32_t o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float v0 = acc[r][c][8 * h + 2 * e], v1 = acc[r][c][8 * h + 2 * e + 1];
+                    if (MODE == BLOCKWISE) {
+                        v0 *= f_out;
+                        v1 *= f_out;
+                    }
+                    if (MODE == ROWCOL) {
+                        const uint32_t bw = e == 0 ? bias[c][h].x : e == 1 ? bias[c][h].y
+                                          : e == 2 ? bias[c][h].z : bias[c][h].w;
+                        v0 = fmaf(v0, sam[r] * sbv[c][h][2 * e], bf16_bits_to_f32(bw & 0xffffu));
+                        v1 = fmaf(v1, sam[r] * sbv[c][h][2 * e + 1], bf16_bits_to_f32(bw >> 16));
+                    }
+                    o[e] = pack_bf16(v0, v1);
+                    if (ACT == HN_ACT_GELU_TANH) {
+                        if (round_first) {
+                            v0 = __uint_as_float(o[e] << 16);
+                            v1 = __uint_as_float(o[e] & 0xffff0000u);
+                        }
+                        o[e] = pack_bf16(gelu_tanh(v0), gelu_tanh(v1));
+                    }
+                }
+                *reinterpret_cast<uint4*>(p.out + m * p.ldc + n) = make_uint4(o[0], o[1], o[2], o[3]);
+            }
+    }
+}
+
 }  // namespace gemm
 }  // namespace hn
 
 using namespace hn;
+
+// The launch of gemm_small_kernel.
+template <int MODE, int WR, int WC, int RB, int CB>
+static void launch_small_as(gemm::Params p, hipStream_t st) {
+    constexpr int TM = 32 * WR * RB, TN = 32 * WC * CB, LDS = gemm::small_stages(TM, TN) * gemm::small_stage_bytes(TM, TN);
+    p.tiles_m = (int)((p.M + TM - 1) / TM);
+    p.tiles_n = (int)((p.N + TN - 1) / TN);
+    p.per_xcd = (int)(((int64_t)p.tiles_m * p.tiles_n + 7) / 8);
+    // The n tiles that an XCD runs at once read g TM rows of A and (n / g) TN of
+    // B: least at g = sqrt(n TN / TM), here with the groups evened out.
+    const double n = std::min(p.per_xcd, 32), g = std::sqrt(n * TN / TM);
+    const int groups = std::max(1, (int)std::lround(p.tiles_m / std::max(1.0, g)));
+    p.group = (p.tiles_m + groups - 1) / groups;
+    const dim3 grid((unsigned)(8 * (int64_t)p.per_xcd)), block(64 * WR * WC);
+    // Below O_MIN_KT steps GELU acts on the fp32 value, elsewhere on its bf16
+    // rounding (as in the persistent kernel).
+    const int round_first = p.K / gemm::BK >= gemm::O_MIN_KT;
+    if constexpr (MODE == gemm::BLOCKWISE)
+        gemm::gemm_small_kernel<MODE, HN_ACT_NONE, WR, WC, RB, CB><<<grid, block, LDS, st>>>(p, 0);
+    else if (p.act == HN_ACT_GELU_TANH)
+        gemm::gemm_small_kernel<MODE, HN_ACT_GELU_TANH, WR, WC, RB, CB><<<grid, block, LDS, st>>>(p, round_first);
+    else
+        gemm::gemm_small_kernel<MODE, HN_ACT_NONE, WR, WC, RB, CB><<<grid, block, LDS, st>>>(p, 0);
+}
+
+// The tile of a launch, by an estimate of each shape's time in us:
+//     3 + rounds * (g + K steps * c),
+// with rounds the number of tiles per CU, rounded up (64 x 64 tiles run two to
+// a CU: 0.3 more instead), and g (a tile's prologue and epilogue) and c (a
+// K step) between their values for a few tiles and for a tile on every CU,
+// where the loads from the L2s (11-15 TB/s in all) and the output's writes
+// bound them. Fitted to back-to-back calls at K 512 to 12288 and 32 to 4608
+// tiles; within 15 % of them, except where the weight comes from HBM.
+struct TileCost {
+    int tm, tn;
+    float g_low, c_low, g_full, c_full;
+};
+
+static double tile_time(const TileCost& t, int64_t M, int64_t N, int64_t K, int cus) {
+    const double tiles = (double)((M + t.tm - 1) / t.tm) * (double)((N + t.tn - 1) / t.tn);
+    const double fill = std::min(1.0, tiles / cus);
+    const double rounds = t.tm * t.tn <= 64 * 64 && tiles > cus ? tiles / cus + 0.3 : std::ceil(tiles / cus);
+    const double g = t.g_low + (t.g_full - t.g_low) * fill, c = t.c_low + (t.c_full - t.c_low) * fill;
+    return 3.0 + rounds * (g + (double)(K / gemm::BK) * c);
+}
+
+// gemm_small_kernel's shapes, per mode.
+constexpr TileCost kSmallRowcol[] = {
+    {64, 64, 1.3f, 0.18f, 1.3f, 0.18f},   {64, 128, 1.2f, 0.27f, 2.0f, 0.38f},
+    {128, 128, 2.5f, 0.34f, 2.5f, 0.60f}, {128, 192, 2.5f, 0.43f, 3.0f, 0.75f},
+    {128, 256, 2.0f, 0.57f, 4.5f, 0.86f}, {256, 192, 0.5f, 0.90f, 7.2f, 1.08f}};
+constexpr TileCost kSmallBlockwise[] = {
+    {64, 64, 1.0f, 0.25f, 1.0f, 0.25f}, {128, 128, 1.0f, 0.48f, 1.0f, 0.62f}, {128, 256, 1.4f, 0.75f, 2.0f, 1.02f}};
+// The 256 x 256 tiles of gemm_rowcol_oe_kernel (its prologues and epilogues
+// run beside other tiles' K steps, all but kBigOnce of them) and gemm_bw8_kernel.
+constexpr TileCost kBigRowcol = {256, 256, 0.0f, 1.12f, 0.0f, 1.52f};
+constexpr TileCost kBigBlockwise = {256, 256, 1.0f, 1.20f, 0.0f, 1.72f};
+constexpr double kBigOnce = 4.0;
+
+// The index of the small tile that a launch takes, or -1 for the 256 x 256
+// tiles. Below O_MIN_KT steps the persistent kernel cannot run. A last stripe
+// of at most TAIL_ROWS rows costs the 256 x 256 tiles no round. Within 3 % of
+// each other the 256 x 256 tiles win.
+static int small_plan(int mode, int64_t M, int64_t N, int64_t K, int cus) {
+    const bool row = mode == gemm::ROWCOL;
+    if (M <= gemm::TAIL_ROWS && K / gemm::BK >= (row ? gemm::O_MIN_KT : 4)) return -1;  // the tail kernel alone
+    const TileCost* const t = row ? kSmallRowcol : kSmallBlockwise;
+    const int count = row ? (int)std::size(kSmallRowcol) : (int)std::size(kSmallBlockwise);
+    int best = 0;
+    for (int i = 1; i < count; ++i)
+        if (tile_time(t[i], M, N, K, cus) < tile_time(t[best], M, N, K, cus)) best = i;
+    if (row && K / gemm::BK < gemm::O_MIN_KT) return best;
+    const int64_t tail = M % gemm::BM, Mb = tail <= gemm::TAIL_ROWS && M > tail ? M - tail : M;
+    const double big = kBigOnce + tile_time(row ? kBigRowcol : kBigBlockwise, Mb, N, K, cus);
+    return tile_time(t[best], M, N, K, cus) < 0.97 * big ? best : -1;
+}
+
+static int launch_small(const gemm::Params& p, int mode, int i, void* stream, const char* who) {
+    const hipStream_t st = (hipStream_t)stream;
+    if (mode == gemm::BLOCKWISE) {
+        if (i == 0) launch_small_as<gemm::BLOCKWISE, 2, 2, 1, 1>(p, st);
+        else if (i == 1) launch_small_as<gemm::BLOCKWISE, 4, 2, 1, 2>(p, st);
+        else launch_small_as<gemm::BLOCKWISE, 2, 4, 2, 2>(p, st);
+    } else {
+        switch (i) {
+            case 0: launch_small_as<gemm::ROWCOL, 2, 2, 1, 1>(p, st); break;
+            case 1: launch_small_as<gemm::ROWCOL, 2, 4, 1, 1>(p, st); break;
+            case 2: launch_small_as<gemm::ROWCOL, 4, 2, 1, 2>(p, st); break;
+            case 3: launch_small_as<gemm::ROWCOL, 4, 2, 1, 3>(p, st); break;
+            case 4: launch_small_as<gemm::ROWCOL, 2, 4, 2, 2>(p, st); break;
+            default: launch_small_as<gemm::ROWCOL, 4, 2, 2, 3>(p, st); break;
+        }
+    }
+    return check_launch(who);
+}
 
 static int gemm_launch(int mode, const void* a, const void* b, const float* sa, const float* sb,
                        const void* bias, void* out, int64_t M, int64_t N, int64_t K, int64_t ldc,
@@ -1634,9 +1738,10 @@ static int gemm_launch(int mode, const void* a, const void* b, const float* sa, 
     p.bias = (const uint16_t*)bias;
     p.out = (uint16_t*)out;
     p.M = M; p.N = N; p.K = K; p.ldc = ldc; p.act = act;
-    HN_REQUIRE((M + gemm::BM - 1) / gemm::BM * ((N + 191) / 192) <= 0x7fffffffLL, HN_E_ARG,
+    HN_REQUIRE((M + 63) / 64 * (N / 64) <= 0x7ffffff0LL, HN_E_ARG,
                "FP8 GEMM: too many tiles");
-    const bool persistent = mode == gemm::ROWCOL && K / gemm::BK >= gemm::O_MIN_KT;
+    if (const int i = small_plan(mode, M, N, K, device_cus()); i >= 0) return launch_small(p, mode, i, stream, who);
+    const bool persistent = mode == gemm::ROWCOL;  // K has at least O_MIN_KT steps here
     // A last row stripe of at most TAIL_ROWS rows goes to gemm_tail_kernel (or,
     // in persistent launches, possibly to the light workgroups), and the tiles
     // cover only the rows above it: always in persistent launches; in
@@ -1657,15 +1762,11 @@ static int gemm_launch(int mode, const void* a, const void* b, const float* sa, 
     }
     const int64_t Mt = stripe ? M - m_tail : M;
     const int64_t tm = (Mt + gemm::BM - 1) / gemm::BM;
-    auto set_tiles = [&](int bn) {
-        const gemm::TileCounts t = gemm::tile_counts(Mt, N, bn);
-        p.bn = bn;
-        p.tiles_m = t.tiles_m; p.tiles_n = t.tiles_n;
-        p.tm_full = t.tm_full; p.tn_full = t.tn_full; p.m_tail = t.m_tail;
-        p.tiles_full = t.tiles_full; p.tiles_part = t.tiles_part;
-        p.per_xcd = mode == gemm::ROWCOL ? t.per_xcd : (int)((tm * t.tiles_n + 7) / 8);
-    };
-    set_tiles(gemm::BN);
+    const gemm::TileCounts t = gemm::tile_counts(Mt, N, gemm::BN);
+    p.tiles_m = t.tiles_m; p.tiles_n = t.tiles_n;
+    p.tm_full = t.tm_full; p.tn_full = t.tn_full; p.m_tail = t.m_tail;
+    p.tiles_full = t.tiles_full; p.tiles_part = t.tiles_part;
+    p.per_xcd = mode == gemm::ROWCOL ? t.per_xcd : (int)((tm * t.tiles_n + 7) / 8);
     const dim3 grid((unsigned)(8 * (int64_t)p.per_xcd));
     // The tail stripe on a launch of its own, with the full M for its row
     // clamp and stores. K is split over 2 waves, or 4 when the stripe has
@@ -1699,17 +1800,8 @@ static int gemm_launch(int mode, const void* a, const void* b, const float* sa, 
     p.tail_M = Mt;
     if (persistent) {
         // Persistent: per XCD, min(queue length, CUs of the XCD) workgroups.
-        // A launch of fewer 256-wide tiles than CUs is one round whatever
-        // the tile; 192-wide tiles (three 32-column blocks per wave) do 3/4
-        // of the work each and fill more CUs (config 1, 4096 x 3072: 192 ->
-        // 256 tiles).
         const int cus = device_cus();
         const int per_xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
-        const int64_t t256 = tm * ((N + 255) / 256), t192 = tm * ((N + 191) / 192);
-        if (t256 < cus && t192 > t256) {
-            set_tiles(192);
-            if (p.per_xcd > per_xcd_cus) set_tiles(gemm::BN);  // would need a second round
-        }
         int wg_cap = per_xcd_cus;
 #ifdef HN_GEMM_PHASE_STAMPS
         // Measurement build: HN_GEMM_WG_PER_XCD caps the workgroups per XCD
@@ -1739,18 +1831,8 @@ static int gemm_launch(int mode, const void* a, const void* b, const float* sa, 
                 return rc;
             }
         }
-        if (p.bn == 192) {
-            if (act == HN_ACT_GELU_TANH)
-                gemm::gemm_rowcol_oe_kernel<HN_ACT_GELU_TANH, 96><<<pgrid, gemm::NT, 0, st>>>(p);
-            else
-                gemm::gemm_rowcol_oe_kernel<HN_ACT_NONE, 96><<<pgrid, gemm::NT, 0, st>>>(p);
-        } else if (act == HN_ACT_GELU_TANH) {
-            gemm::gemm_rowcol_oe_kernel<HN_ACT_GELU_TANH, 128><<<pgrid, gemm::NT, 0, st>>>(p);
-        } else {
-            gemm::gemm_rowcol_oe_kernel<HN_ACT_NONE, 128><<<pgrid, gemm::NT, 0, st>>>(p);
-        }
-    } else if (mode == gemm::ROWCOL) {
-        gemm::gemm_rowcol_kernel<<<grid, gemm::NT, 0, (hipStream_t)stream>>>(p);
+        if (act == HN_ACT_GELU_TANH) gemm::gemm_rowcol_oe_kernel<HN_ACT_GELU_TANH><<<pgrid, gemm::NT, 0, st>>>(p);
+        else gemm::gemm_rowcol_oe_kernel<HN_ACT_NONE><<<pgrid, gemm::NT, 0, st>>>(p);
     } else {
         if (stripe) {
             if (const int rc = launch_tail(); rc != HN_OK) return rc;

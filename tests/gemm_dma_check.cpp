@@ -152,7 +152,55 @@ static int tailwide_main(int argc, char** argv) {
     return 0;
 }
 
+// gemm_small_kernel: every tile of a launch once, and every load of every wave
+// and K step inside its operand (rows inside it at their exact offsets, rows
+// past it on its last row).
+static int small_main(int argc, char** argv) {
+    if (argc != 9) {
+        fprintf(stderr, "usage: %s small M N K TM TN WAVES GROUP\n", argv[0]);
+        return 2;
+    }
+    const int64_t M = atoll(argv[2]), N = atoll(argv[3]), K = atoll(argv[4]);
+    const int TM = atoi(argv[5]), TN = atoi(argv[6]), waves = atoi(argv[7]), group = atoi(argv[8]);
+    const int tiles_m = (int)((M + TM - 1) / TM), tiles_n = (int)((N + TN - 1) / TN);
+    const int nq = (TM + TN) / (8 * waves);
+    if (M <= 0 || N <= 0 || K % 128 || group < 1 || nq * 8 * waves != TM + TN) {
+        fprintf(stderr, "bad shape\n");
+        return 2;
+    }
+    long long loads = 0, oob = 0, wrong = 0, cover = 0;
+    int* hits = (int*)calloc((size_t)tiles_m * tiles_n, sizeof(int));
+    for (int item = 0; item < tiles_m * tiles_n; ++item) {
+        int tm = -1, tn = -1;
+        small_tile(item, tiles_m, tiles_n, group, tm, tn);
+        if (tm < 0 || tm >= tiles_m || tn < 0 || tn >= tiles_n) {
+            ++cover;
+            continue;
+        }
+        ++hits[tm * tiles_n + tn];
+        const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
+        for (int q = 0; q < waves * nq; ++q)
+            for (int lane = 0; lane < 64; ++lane) {
+                const TailSrc ts = tail_wide_src(q, lane, TM, m0, M, n0, N - 1, K);
+                const int row = 8 * q + (lane >> 3);
+                const int64_t extent = ts.a ? M : N, at = ts.a ? m0 + row : n0 + row - TM;
+                const int64_t chunk = (int64_t)swz_pos(row, lane & 7) * 16;
+                if (ts.a != (row < TM) || ts.off != (at < extent ? at : extent - 1) * K + chunk) ++wrong;
+                for (int64_t st = 0; st < K / 128; ++st) {
+                    const int64_t addr = ts.off + st * 128;
+                    ++loads;
+                    if (addr < 0 || addr + 16 > extent * K) ++oob;
+                }
+            }
+    }
+    for (int i = 0; i < tiles_m * tiles_n; ++i) cover += hits[i] != 1;
+    free(hits);
+    printf("loads=%lld out_of_bounds=%lld wrong_offset=%lld tile_cover_errors=%lld\n", loads, oob, wrong, cover);
+    return 0;
+}
+
 int main(int argc, char** argv) {
+    if (argc > 1 && strcmp(argv[1], "small") == 0) return small_main(argc, argv);
     if (argc > 1 && strcmp(argv[1], "tail") == 0) return tail_main(argc, argv);
     if (argc > 1 && strcmp(argv[1], "tailwide") == 0) return tailwide_main(argc, argv);
     if (argc < 5) {

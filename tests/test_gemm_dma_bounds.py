@@ -107,3 +107,17 @@ def test_tail_items_on_light_workgroups(checker, M, N, K, cus, fused):
     if fused:
         assert r["loads"] > 0 and r["out_of_bounds"] == 0 and r["wrong_offset"] == 0, r
         assert r["column_cover_errors"] == 0 and r["not_light"] == 0 and r["cols"] <= 384, r
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (100, 384, 256), (257, 640, 384), (1025, 1152, 128)])
+@pytest.mark.parametrize("TM,TN,waves", [(64, 64, 4), (64, 128, 8), (128, 128, 8), (128, 192, 8), (128, 256, 8),
+                                         (256, 192, 8)])
+def test_small_tile_loads_stay_inside(checker, M, N, K, TM, TN, waves):
+    """The small-tile kernel's shapes: every tile exactly once whatever the
+    group size, every load in bounds and on its row."""
+    for group in (1, 3, 7, 64):
+        out = subprocess.run([str(checker), "small", *map(str, (M, N, K, TM, TN, waves, group))], check=True,
+                             capture_output=True, text=True).stdout
+        r = {k: int(v) for k, v in (kv.split("=") for kv in out.split())}
+        assert r["loads"] > 0 and r["out_of_bounds"] == 0 and r["wrong_offset"] == 0, r
+        assert r["tile_cover_errors"] == 0, r

@@ -430,3 +430,39 @@ def test_fp8_linear_modules(O, dev):
     assert_close_bf16(y2.reshape(-1, 128).float().cpu().numpy(), ref2, what="FP8StoredLinear")
     with pytest.raises(TypeError):
         d(x.float())
+
+
+# Launches that take each shape of the small-tile kernel on 256 CUs, ragged in M
+# and (192- and 256-wide tiles) in N; K of 5 to 9 steps covers the pipeline's
+# fill and drain, and K below 896 the GELU of the unrounded value.
+@pytest.mark.parametrize("M,K,N", [
+    (100, 1024, 256), (65, 128, 384),       # 64 x 64
+    (450, 1024, 3200), (1000, 768, 2048),   # 64 x 128
+    (1000, 1024, 3072),                     # 128 x 128
+    (1025, 896, 4224),                      # 128 x 192
+    (2049, 896, 2944), (4097, 640, 3200),   # 128 x 256
+    (3000, 896, 3072), (2500, 640, 4224),   # 256 x 192
+])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear_fp8_small_tiles(O, dev, M, K, N, gelu):
+    print(f"case small tiles {M}x{K}x{N} gelu={gelu}", flush=True)
+    rows = np.unique(np.concatenate([np.arange(0, min(M, 160)), np.arange(max(0, M - 160), M)]))
+    _check_linear(O, dev, M, K, N, gelu, bias=not gelu, rows=rows)
+
+
+@pytest.mark.parametrize("m,n,k", [(129, 256, 384), (1000, 1024, 2048), (2200, 640, 1920)])
+def test_blockwise_gemm_small_tiles(O, dev, m, n, k):
+    """The blockwise small tiles (64 x 64, 128 x 128, 128 x 256) with K blocks of
+    gains up to 2^+-8, an all-zero activation block and zero factors."""
+    print(f"case blockwise small tiles {m}x{n}x{k}", flush=True)
+    pf = pkg_module("pixelumm_fp8")
+    g = torch.Generator().manual_seed(m + n)
+    gain = 2.0 ** torch.randint(-8, 9, (k // 128,), generator=g).float()
+    a = torch.randn(m, k, generator=g) * gain.repeat_interleave(128)[None, :]
+    a[:, 128:256] = 0.0
+    qa, sa = pf._quantize_blockwise(a.to(torch.bfloat16).to(dev))
+    qb, sb = pf._quantize_blockwise(torch.randn(n, k, generator=g).to(torch.bfloat16).to(dev))
+    sb[0, 0] = 0.0     # the first K block of the first columns
+    sa[-1, -1] = 0.0   # the last K block of the last rows
+    expected = O.blockwise_gemm_reference(u8(qa), sa.cpu().numpy(), u8(qb), sb.cpu().numpy())
+    _blockwise_check(pf.load_extension().gemm(qa, qb, sa, sb), expected)
