@@ -150,18 +150,12 @@ HN_DEVICE uint32_t pack_f16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, f16x2));
 }
 
-// fp16 bits of the two bf16 values of word w (lo, hi), packed (lo low). Exact
-// for bf16 values in fp16's range; round toward zero, so magnitudes past
-// 65504 saturate instead of overflowing.
-HN_DEVICE uint32_t bf16x2_to_f16x2(uint32_t w) {
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(bf16_lo(w), bf16_hi(w)));
-}
-
 // fp16 bits of bf16(a), bf16(b): the reference's bf16 dequantized values held
 // as fp16 operands of the PV MFMA. Each value is rounded as the high half of a
 // pair whose low half is 0, which is the fp32 form of its bf16 value as it
 // stands: 3 instructions for two values, where rounding them as one pair and
-// taking it apart again costs 4.
+// taking it apart again costs 4. Exact for bf16 values in fp16's normal range;
+// the pack rounds toward zero, so magnitudes past 65504 saturate.
 HN_DEVICE uint32_t pack_f16_of_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(__uint_as_float(pack_bf16(0.0f, a)),
                                                                    __uint_as_float(pack_bf16(0.0f, b))));
@@ -465,21 +459,27 @@ HN_DEVICE void load_tail_k(const Params& p, int64_t b, int64_t h, int64_t first,
 }
 
 template <int NW, bool MASK>
-HN_DEVICE void store_tail_k(const TailRegs<NW>& r, uint8_t* st) {
-    const int t = threadIdx.x;
+HN_DEVICE void store_tail_mask(const TailRegs<NW>& r, uint8_t* st) {
     if constexpr (MASK) {
-        if ((t >> 6) == 2) {
+        if ((threadIdx.x >> 6) == 2) {
             const uint64_t bits = __ballot(r.mk != 0u);
-            if ((t & 63) == 0) *reinterpret_cast<uint64_t*>(st + MASK_OFF) = bits;
+            if ((threadIdx.x & 63) == 0) *reinterpret_cast<uint64_t*>(st + MASK_OFF) = bits;
         }
     }
+}
+
+// 16-byte half `hf` of unit i's 32 bytes.
+template <int NW>
+HN_DEVICE void store_tail_k_part(const TailRegs<NW>& r, uint8_t* st, int i, int hf) {
+    const int key = (int)k_key(threadIdx.x) + (Shape<NW>::NT / 8) * i;
+    reinterpret_cast<uint4*>(st + key * KROW + (int)k_unit(threadIdx.x) * 32)[hf] = r.k[2 * i + hf];
+}
+
+template <int NW, bool MASK>
+HN_DEVICE void store_tail_k(const TailRegs<NW>& r, uint8_t* st) {
+    store_tail_mask<NW, MASK>(r, st);
 #pragma unroll
-    for (int i = 0; i < Shape<NW>::KU; ++i) {
-        const int key = (int)k_key(t) + (Shape<NW>::NT / 8) * i, unit = (int)k_unit(t);
-        uint4* dst = reinterpret_cast<uint4*>(st + key * KROW + unit * 32);
-        dst[0] = r.k[2 * i];
-        dst[1] = r.k[2 * i + 1];
-    }
+    for (int i = 0; i < 2 * Shape<NW>::KU; ++i) store_tail_k_part<NW>(r, st, i >> 1, i & 1);
 }
 
 template <int NW>
@@ -500,20 +500,73 @@ HN_DEVICE void load_tail_v(const Params& p, int64_t b, int64_t h, int64_t first,
     }
 }
 
-// V^T holds fp16: the bf16 values converted (exactly, in fp16's range).
+// V^T holds fp16: the bf16 values converted (exactly, in fp16's range). Part d:
+// the thread's dim d, 4 keys.
 template <int NW>
-HN_DEVICE void store_tail_v(const TailRegs<NW>& r, uint8_t* st) {
+HN_DEVICE void store_tail_v_part(const TailRegs<NW>& r, uint8_t* st, int d) {
     constexpr int VD = Shape<NW>::VD;
     const int qd = threadIdx.x & 15, dg = v_group<NW>();
+    uint32_t o[2];
 #pragma unroll
-    for (int d = 0; d < VD; ++d) {
-        uint32_t o[2];
-        const uint32_t sh = (d & 1) * 16;
+    for (int pr = 0; pr < 2; ++pr) {
+        const uint32_t a = r.v[2 * pr][d >> 1], b = r.v[2 * pr + 1][d >> 1];
+        o[pr] = __builtin_bit_cast(uint32_t, (d & 1) ? __builtin_amdgcn_cvt_pkrtz(bf16_hi(a), bf16_hi(b))
+                                                     : __builtin_amdgcn_cvt_pkrtz(bf16_lo(a), bf16_lo(b)));
+    }
+    *reinterpret_cast<uint2*>(st + K_BYTES + (VD * dg + d) * VTROW + 8 * qd) = make_uint2(o[0], o[1]);
+}
+
+template <int NW>
+HN_DEVICE void store_tail_v(const TailRegs<NW>& r, uint8_t* st) {
 #pragma unroll
-        for (int pr = 0; pr < 2; ++pr)
-            o[pr] = bf16x2_to_f16x2(((r.v[2 * pr][d >> 1] >> sh) & 0xffffu) |
-                                    (((r.v[2 * pr + 1][d >> 1] >> sh) & 0xffffu) << 16));
-        *reinterpret_cast<uint2*>(st + K_BYTES + (VD * dg + d) * VTROW + 8 * qd) = make_uint2(o[0], o[1]);
+    for (int d = 0; d < Shape<NW>::VD; ++d) store_tail_v_part<NW>(r, st, d);
+}
+
+// Steady tail tiles: loads through descriptors spanning the (batch, head) tail
+// rows [0, tail_end), at the tile's byte offset `co` (rows past the end read as
+// zeros), with the lane's offsets inside a tile.
+template <int NW>
+struct TailOffs {
+    uint32_t k[Shape<NW>::KU], v[4];
+};
+
+template <int NW>
+HN_DEVICE TailOffs<NW> tail_offsets(const Params& p) {
+    TailOffs<NW> o;
+    const uint32_t t = threadIdx.x, pitch = 2 * (uint32_t)p.us1;
+#pragma unroll
+    for (int i = 0; i < Shape<NW>::KU; ++i)
+        o.k[i] = (k_key(t) + (uint32_t)(Shape<NW>::NT / 8) * i) * pitch + k_unit(t) * 32u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        o.v[j] = (uint32_t)quad_key(t & 15, j) * pitch + (uint32_t)(2 * Shape<NW>::VD * v_group<NW>());
+    return o;
+}
+
+template <int NW, bool MASK>
+HN_DEVICE void load_tail_span_k(const Params& p, int64_t b, const TailOffs<NW>& lo, __amdgpu_buffer_rsrc_t k,
+                                uint32_t co, int64_t first, int64_t end, TailRegs<NW>& r) {
+    if constexpr (MASK) {
+        if ((threadIdx.x >> 6) == 2) {
+            const int64_t j = first + (threadIdx.x & 63);
+            r.mk = j < end ? (p.uvalid ? (uint32_t)p.uvalid[b * p.uvs + j] : 1u) : 0u;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < Shape<NW>::KU; ++i) {
+        r.k[2 * i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(k, lo.k[i] + co, 0, 0));
+        r.k[2 * i + 1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(k, lo.k[i] + co + 16, 0, 0));
+    }
+}
+
+template <int NW>
+HN_DEVICE void load_tail_span_v(const TailOffs<NW>& lo, __amdgpu_buffer_rsrc_t v, uint32_t co, TailRegs<NW>& r) {
+    static_assert(Shape<NW>::VD == 4, "two dwords per key");
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(v, lo.v[j] + co, 0, 0));
+        r.v[j][0] = x.x;
+        r.v[j][1] = x.y;
     }
 }
 
@@ -605,6 +658,22 @@ HN_DEVICE float mask_raw(f32x16& u, int kb, int half, int lim, uint64_t mw) {
     return mx;
 }
 
+// A block whose keys' validity is the same for every query: bit j of w is key j
+// of the block. The two halves of the wave hold different keys, so register v's
+// lane mask is one bit of w for lanes 0-31 and another for lanes 32-63, made by
+// scalar instructions: one select per logit, where mask_raw's per-lane bit and
+// limit tests take about four more. Returns the new max. 7712 masked queries
+// over 14 912 keys with 2 % holes: 1.980 -> 1.970 ms.
+HN_DEVICE float mask_word(f32x16& u, uint32_t w) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int j = 8 * (v >> 2) + (v & 3);
+        const uint64_t lo = (w >> j) & 1u ? 0xffffffffull : 0ull, hi = (w >> (j + 4)) & 1u ? 0xffffffffull : 0ull;
+        u[v] = __builtin_amdgcn_inverse_ballot_w64(hi << 32 | lo) ? u[v] : -INFINITY;
+    }
+    return raw_max(u);
+}
+
 // Before a block's probabilities, with the lane's raw block max mx (its
 // logit max in log2 units is mx * c, c = softmax_scale * log2 e > 0): taken,
 // wave-uniformly, only when some lane's logit max passes m + REBASE_SLACK
@@ -688,24 +757,15 @@ HN_DEVICE f32x16 step_a(const f32x16& s, float c, float nm, float& l, f16x8 (&pf
 
 // Step B: O^T += V^T P^T of block kb (V^T operand reads at va: this lane's
 // row and column in the stage) beside the raw max of the next block (s) and,
-// per STORE (1: K, 2: V^T), half of the write of the prefetched tile to stage
-// nst with the scales of buffer sb. Returns the next block's raw max over this
-// lane's keys.
-template <int FMT, int NW, int STORE>
-HN_DEVICE float step_b(const f16x8 (&pf)[2], const uint8_t* va, int kb, f32x16 (&o)[4], const f32x16& s,
-                       const CacheRegs<NW>& r, uint8_t* nst, const float* sb) {
+// in slot i, beside(i). Returns the next block's raw max over this lane's keys.
+template <typename F>
+HN_DEVICE float step_b_with(const f16x8 (&pf)[2], const uint8_t* va, int kb, f32x16 (&o)[4], const f32x16& s,
+                            F beside) {
     // operand i (= 4 tt + db): dim block db, 16-key slice 2 kb + tt
     f16x8 vf[8];
     vf[0] = ld_f16x8(va + 64 * kb);
     vf[1] = ld_f16x8(va + 64 * kb + 32 * VTROW);
-    float ks[Shape<NW>::KU] = {};
-    float4 vs = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (STORE == 1) k_scales<NW>(sb, ks);
-    if (STORE == 2) vs = v_scales(sb);
     float mx = -INFINITY;
-    uint32_t kd[4];
-    float vp[Shape<NW>::VD];
-    uint32_t vd[2 * Shape<NW>::VD];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int tt = i >> 2, db = i & 3;
@@ -716,11 +776,28 @@ HN_DEVICE float step_b(const f16x8 (&pf)[2], const uint8_t* va, int kb, f32x16 (
         o[db] = mfma_f16(vf[i], pf[tt], o[db]);
         mx = fmaxf(mx, fmaxf(s[2 * i], s[2 * i + 1]));
         pin(mx);
-        if (STORE == 1) store_k_part<FMT, NW>(r, nst, i, ks, kd);
-        if (STORE == 2) store_v_part<FMT, NW>(r.v, nst + K_BYTES, i, vs, vp, vd);
+        beside(i);
         __builtin_amdgcn_sched_barrier(0);
     }
     return mx;
+}
+
+// Step B beside half of the write of the prefetched cache tile (STORE 1: K, 2:
+// V^T) to stage nst with the scales of buffer sb.
+template <int FMT, int NW, int STORE>
+HN_DEVICE float step_b(const f16x8 (&pf)[2], const uint8_t* va, int kb, f32x16 (&o)[4], const f32x16& s,
+                       const CacheRegs<NW>& r, uint8_t* nst, const float* sb) {
+    float ks[Shape<NW>::KU] = {};
+    float4 vs = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (STORE == 1) k_scales<NW>(sb, ks);
+    if (STORE == 2) vs = v_scales(sb);
+    uint32_t kd[4];
+    float vp[Shape<NW>::VD];
+    uint32_t vd[2 * Shape<NW>::VD];
+    return step_b_with(pf, va, kb, o, s, [&](int i) __attribute__((always_inline)) {
+        if (STORE == 1) store_k_part<FMT, NW>(r, nst, i, ks, kd);
+        if (STORE == 2) store_v_part<FMT, NW>(r.v, nst + K_BYTES, i, vs, vp, vd);
+    });
 }
 
 template <int FMT, int NW, bool MASK>
@@ -846,6 +923,17 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
         lim64 = lim64 < g.count ? lim64 : g.count;
         return lim64 < 0 ? 0 : (int)lim64;
     };
+    // Masks block kb of tile g, whose validity word is mw, where something is to
+    // mask; mx: the block's unmasked max. Without chunks a limit is the same
+    // for every query, so it joins the word.
+    auto mask_block = [&](f32x16& u, int kb, const Geom& g, uint64_t mw, float mx) {
+        if (g.full || p.chunk == 0) {
+            const uint64_t all = g.count >= BKV ? ALL_KEYS : (1ull << g.count) - 1;
+            const uint32_t w = (uint32_t)((mw & all) >> (32 * kb));
+            return w == ~0u ? mx : mask_word(u, w);
+        }
+        return mask_raw(u, kb, half, lim_of(g), mw);
+    };
     // This lane's K row (block 0) at dims 8 half .., and its V^T row (dim
     // block 0) at column unit `half` (slice 0).
     const uint32_t ka_off = col * KROW + 16 * half;
@@ -930,7 +1018,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 mw = tile_mask<MASK>(smem);
                 sa = s_block(smem + ka_off, qf);
                 mxa = raw_max(sa);
-                if (!g.full || mw != ALL_KEYS) mxa = mask_raw(sa, 0, half, lim_of(g), mw);
+                if (!g.full || mw != ALL_KEYS) mxa = mask_block(sa, 0, g, mw, mxa);
             }
             int t = t_begin;
             {
@@ -950,7 +1038,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                     mxb = step_b<FMT, NW, 1>(pf, st + va_off, 0, o, sb, regs, nst, nsb);
                     if constexpr (MASK) {
                         store_mask<NW, MASK>(regs, nst);
-                        if (mw != ALL_KEYS) mxb = mask_raw(sb, 1, half, BKV, mw);
+                        if ((uint32_t)(mw >> 32) != ~0u) mxb = mask_word(sb, (uint32_t)(mw >> 32));
                     }
                     load_k<NW, MASK>(lo, regs, span, BKV, fco, fso, (int64_t)(t + 2) * BKV);
                     __syncthreads();
@@ -959,7 +1047,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                     mxa = step_b<FMT, NW, 2>(pf, st + va_off, 1, o, sa, regs, nst, nsb);
                     if constexpr (MASK) {
                         mw = tile_mask<MASK>(nst);  // tile t + 1
-                        if (mw != ALL_KEYS) mxa = mask_raw(sa, 0, half, BKV, mw);
+                        if ((uint32_t)mw != ~0u) mxa = mask_word(sa, (uint32_t)mw);
                     }
                     if (threadIdx.x < 2 * BKV) sbuf[(u & 1) * SB_FLOATS + threadIdx.x] = regs.s;
                     load_v<NW>(lo, regs, span, fco);
@@ -988,7 +1076,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 // the stage is not read before the barrier).
                 mxb = step_b<FMT, NW, 1>(pf, st + va_off, 0, o, sb, regs, nst, nsb);
                 store_mask<NW, MASK>(regs, nst);
-                if (!g.full || mw != ALL_KEYS) mxb = mask_raw(sb, 1, half, lim_of(g), mw);
+                if (!g.full || mw != ALL_KEYS) mxb = mask_block(sb, 1, g, mw, mxb);
                 if (has_next && !gn.cache) copy_tail_k<NW, MASK>(p, b, h, gn.first, gn.count, nst);
                 const int n2 = fetch2 && g2.cache ? g2.count : 0;  // 0: no fetch (zeros)
                 load_k<NW, MASK>(lo, regs, tile_base(p, b, h, g2.first, n2), n2);
@@ -1000,7 +1088,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 rebase(mxb, c, run, o);
                 sa = step_a(sb, c, run.nm, run.l, pf, nst + ka_off, qf);
                 mxa = step_b<FMT, NW, 2>(pf, st + va_off, 1, o, sa, regs, nst, nsb);
-                if (!gn.full || mwn != ALL_KEYS) mxa = mask_raw(sa, 0, half, lim_of(gn), mwn);
+                if (!gn.full || mwn != ALL_KEYS) mxa = mask_block(sa, 0, gn, mwn, mxa);
                 if (has_next && !gn.cache) copy_tail_v<NW>(p, b, h, gn.first, gn.count, nst);
                 // (without a fetch: zeros into a scale buffer no write reads)
                 if (threadIdx.x < 2 * BKV) sbuf[(u & 1) * SB_FLOATS + threadIdx.x] = regs.s;
@@ -1058,7 +1146,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
             uint64_t mw = tile_mask<MASK>(smem);  // validity word of tile t
             sa = s_block(smem + ka_off, qf);
             mxa = raw_max(sa);
-                if (!g.full || mw != ALL_KEYS) mxa = mask_raw(sa, 0, half, lim_of(g), mw);
+                if (!g.full || mw != ALL_KEYS) mxa = mask_block(sa, 0, g, mw, mxa);
             int t = t_begin;
             {
                 // steady tiles (see t_fast): fetch tile t + NS at offsets fco / fso
@@ -1081,14 +1169,14 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                     mxb = step_b<FMT, NW, 1>(pf, st + va_off, 0, o, sb, regs, wst, wsb);
                     if constexpr (MASK) {
                         store_mask<NW, MASK>(regs, wst);
-                        if (mw != ALL_KEYS) mxb = mask_raw(sb, 1, half, BKV, mw);
+                        if ((uint32_t)(mw >> 32) != ~0u) mxb = mask_word(sb, (uint32_t)(mw >> 32));
                     }
                     load_k<NW, MASK>(lo, regs, span, BKV, fco, fso, (int64_t)(t + NS) * BKV);
                     rebase(mxb, c, run, o);
                     sa = step_a(sb, c, run.nm, run.l, pf, st1 + ka_off, qf);
                     mxa = step_b<FMT, NW, 2>(pf, st + va_off, 1, o, sa, regs, wst, wsb);
                     if constexpr (MASK) {
-                        if (mwn != ALL_KEYS) mxa = mask_raw(sa, 0, half, BKV, mwn);
+                        if ((uint32_t)mwn != ~0u) mxa = mask_word(sa, (uint32_t)mwn);
                         mw = mwn;
                     }
                     if (threadIdx.x < 2 * BKV) sbuf[((u + NS) & 1) * SB_FLOATS + threadIdx.x] = regs.s;
@@ -1100,7 +1188,15 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 }
                 if (t > t_begin) g = geom(t);
             }
-            for (; t < t_end; ++t) {
+            // The tail's tiles, [t_tail, t_end), run a loop of their own. With the
+            // general loop's geometry, per-lane addresses, unused cache writes and
+            // tail writes after the steps, a tail tile took up to twice a steady
+            // cache tile's time; here it takes less than one (no dequantization).
+            // 11 056 queries over 11 056 cached and 11 056 tail keys with masks, in
+            // the block: 6.09 -> 5.38 ms for the whole block.
+            const bool tail_span = tail_end > 0 && p.us1 > 0 && ((tail_end - 1) * p.us1 + D) * 2 < ((int64_t)1 << 31);
+            const int t_tail = tail_span && t_end > n_cache ? (t > n_cache ? t : n_cache) : t_end;
+            for (; t < t_tail; ++t) {
                 const int u = t - t_begin;
                 const uint8_t* st = smem + (u % NS) * STAGE;              // tile t
                 const uint8_t* st1 = smem + ((u + 1) % NS) * STAGE;       // tile t + 1
@@ -1123,7 +1219,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 // right after: the stage is not read before the barrier).
                 mxb = step_b<FMT, NW, 1>(pf, st + va_off, 0, o, sb, regs, wst, wsb);
                 store_mask<NW, MASK>(regs, wst);
-                if (!g.full || mw != ALL_KEYS) mxb = mask_raw(sb, 1, half, lim_of(g), mw);
+                if (!g.full || mw != ALL_KEYS) mxb = mask_block(sb, 1, g, mw, mxb);
                 if (write && !gw.cache) store_tail_k<NW, MASK>(tregs, wst);
                 const int nf = fetch && gf.cache ? gf.count : 0;  // 0: no fetch (zeros)
                 load_k<NW, MASK>(lo, regs, tile_base(p, b, h, gf.first, nf), nf);
@@ -1134,7 +1230,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 rebase(mxb, c, run, o);
                 sa = step_a(sb, c, run.nm, run.l, pf, st1 + ka_off, qf);
                 mxa = step_b<FMT, NW, 2>(pf, st + va_off, 1, o, sa, regs, wst, wsb);
-                if (!gn.full || mwn != ALL_KEYS) mxa = mask_raw(sa, 0, half, lim_of(gn), mwn);
+                if (!gn.full || mwn != ALL_KEYS) mxa = mask_block(sa, 0, gn, mwn, mxa);
                 if (write && !gw.cache) store_tail_v<NW>(tregs, wst);
                 // (without a fetch: zeros into a scale buffer no write reads)
                 if (threadIdx.x < 2 * BKV) sbuf[((u + NS) & 1) * SB_FLOATS + threadIdx.x] = regs.s;
@@ -1143,6 +1239,45 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 __syncthreads();
                 g = gn;
                 mw = mwn;
+            }
+            if (t < t_end) {
+                const int64_t at = b * p.us0 + h * p.us2, bytes = ((tail_end - 1) * p.us1 + D) * 2;
+                const __amdgpu_buffer_rsrc_t tk = tile_rsrc(p.kcur + at, bytes), tv = tile_rsrc(p.vcur + at, bytes);
+                const TailOffs<NW> to = tail_offsets<NW>(p);
+                uint32_t co = (uint32_t)((int64_t)(t + NS - n_cache) * BKV * p.us1 * 2);
+                const uint32_t dco = (uint32_t)(BKV * p.us1 * 2);
+                // Tiles below t_full exist whole and are visible to every query.
+                const int64_t vis = wg_key_limit - p.kv_len, tail_full = tail_end < vis ? tail_end : vis;
+                const int t_full = n_cache + (tail_full > 0 ? (int)(tail_full / BKV) : 0);
+                int s0 = (t - t_begin) % NS;
+                for (; t < t_end; ++t) {
+                    const int s1 = s0 == NS - 1 ? 0 : s0 + 1, sw = s0 == 0 ? NS - 1 : s0 - 1;
+                    const uint8_t* st = smem + s0 * STAGE;
+                    const uint8_t* st1 = smem + s1 * STAGE;
+                    uint8_t* wst = smem + sw * STAGE;
+                    f16x8 pf[2];
+                    const uint64_t mwn = tile_mask<MASK>(st1);
+                    rebase(mxa, c, run, o);
+                    sb = step_a(sa, c, run.nm, run.l, pf, st + ka_off + 32 * KROW, qf);
+                    mxb = step_b_with(pf, st + va_off, 0, o, sb, [&](int i) __attribute__((always_inline)) {
+                        if (i == 3 || i == 6) store_tail_k_part<NW>(tregs, wst, 0, i == 6);
+                    });
+                    store_tail_mask<NW, MASK>(tregs, wst);
+                    if (t >= t_full || mw != ALL_KEYS) mxb = mask_block(sb, 1, geom(t), mw, mxb);
+                    load_tail_span_k<NW, MASK>(p, b, to, tk, co, (int64_t)(t + NS - n_cache) * BKV, tail_end, tregs);
+                    rebase(mxb, c, run, o);
+                    sa = step_a(sb, c, run.nm, run.l, pf, st1 + ka_off, qf);
+                    mxa = step_b_with(pf, st + va_off, 1, o, sa, [&](int i) __attribute__((always_inline)) {
+                        if (i & 1) store_tail_v_part<NW>(tregs, wst, i >> 1);
+                    });
+                    if (t + 1 >= t_full || mwn != ALL_KEYS)  // (unused on the last tile)
+                        mxa = mask_block(sa, 0, geom(t + 1 < t_end ? t + 1 : t), mwn, mxa);
+                    load_tail_span_v<NW>(to, tv, co, tregs);
+                    __syncthreads();
+                    co += dco;
+                    s0 = s1;
+                    mw = mwn;
+                }
             }
         }
     }

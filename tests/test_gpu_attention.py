@@ -219,6 +219,40 @@ def test_eight_wave_short_key_ranges(O, dev, kv_len, cur_len):
            "8-wave short range")
 
 
+# The 8-wave shape's tail loop: entered from the first tile, from a partial or a
+# whole last cache tile; 1 to 6 tail tiles, whole and partial; K and V strided
+# views of a QKV tensor; key masks; a chunk boundary inside the tail (queries at
+# positions 0 .. 511, chunks of 300).
+@pytest.mark.parametrize("kv_len,cur_len", [(0, 1), (0, 64), (0, 192), (0, 333), (64, 65), (100, 191), (64, 320)])
+@pytest.mark.parametrize("masked,chunk", [(False, 0), (True, 0), (False, 300), (True, 300)])
+def test_eight_wave_tail_tiles(O, dev, kv_len, cur_len, masked, chunk):
+    print(f"case attn 8-wave tail kv={kv_len} cur={cur_len} masked={masked} chunk={chunk}", flush=True)
+    ca = pkg_module("cache_attention")
+    kvc = pkg_module("fp8_kv_cache")
+    H, D, Lq = 128, 128, 512
+    if kv_len:
+        cache = _cache_from_chunks(dev, 1, kv_len, H, D, 40 + kv_len)
+    else:
+        cache = kvc.make_fp8_kv_block(1, 64, H, D, device=dev)
+        for buf in cache.values():
+            buf.view(torch.uint8).zero_()
+    q = _q(dev, Lq, H, D, 43)
+    g = torch.Generator(device=dev).manual_seed(44)
+    qkv = (torch.randn(1, cur_len, 3, H, D, device=dev, generator=g) * 2).to(torch.bfloat16)
+    kc, vc = qkv.select(2, 1), qkv.select(2, 2)
+    n = kv_len + cur_len
+    valid = (torch.rand(1, n, device=dev, generator=g) > 0.3) if masked else torch.ones(1, n, dtype=torch.bool, device=dev)
+    kw = dict(cache_valid=valid[:, :kv_len], cur_valid=valid[:, kv_len:].contiguous()) if masked else {}
+    out = ca.chunk_attention(q, cache, kv_len, k_cur=kc, v_cur=vc, chunk_len=chunk, **kw)
+    kh, vh = _dequant(O, cache, kv_len)
+    kh = np.concatenate([kh, O.bf16_bits_to_f32(bf16_bits(kc[0]))], 0)
+    vh = np.concatenate([vh, O.bf16_bits_to_f32(bf16_bits(vc[0]))], 0)
+    rows = np.concatenate([np.arange(0, Lq, 37), np.arange(298, 302)])
+    vis = O.block_causal_visible(rows, np.arange(n), chunk) if chunk else None
+    _check(O, out[0, rows].float().cpu().numpy(), O.bf16_bits_to_f32(bf16_bits(q[0, rows])), kh, vh,
+           "8-wave tail", visible=vis, key_valid=valid[0].cpu().numpy())
+
+
 @pytest.mark.parametrize("Lq,kv_len,H", [(128, 86400, 24), (100, 20000, 4), (1, 5000, 2)])
 def test_split_kv_decode_style(O, dev, Lq, kv_len, H):
     """Few queries over a long cache: the key range is split across workgroups
