@@ -173,13 +173,20 @@ class FP8DiTBlock(nn.Module):
         GELU-tanh fused into fc1's epilogue, gated residual."""
         B, L, C = x.shape
         with stage("post_fp8"):
-            x = x + fp8_linear(proj, attn.reshape(B, L, C)) * parts[2].unsqueeze(1)
+            y = fp8_linear(proj, attn.reshape(B, L, C))
             if self._fused(fc1):
-                qh, sh = ops.ln_modulate_quantize_fp8(x, parts[3], parts[4], 1e-6)
+                # both residuals in kernels: the first with the LayerNorm and
+                # quantization that follow it
+                x, qh, sh = ops.ln_modulate_quantize_fp8(x, parts[3], parts[4], 1e-6,
+                                                         residual=(y, parts[2].expand(B, C)))
                 h = fp8_linear_codes(fc1, qh, sh, gelu=True).view(B, L, -1)
-            else:
-                h = _modulate(F.layer_norm(x, (C,), eps=1e-6), parts[3], parts[4])
-                h = fp8_linear(fc1, h, gelu=True)
+                h = fp8_linear(fc2, h)
+                if h.dtype == parts[5].dtype == torch.bfloat16:
+                    return ops.gated_residual(x, h, parts[5].expand(B, C))
+                return x + h * parts[5].unsqueeze(1)
+            x = x + y * parts[2].unsqueeze(1)
+            h = _modulate(F.layer_norm(x, (C,), eps=1e-6), parts[3], parts[4])
+            h = fp8_linear(fc1, h, gelu=True)
             h = fp8_linear(fc2, h)
             x = x + h * parts[5].unsqueeze(1)
         return x

@@ -59,15 +59,26 @@ def _(x, scale_mode=L.HN_SCALE_CLAMP, amax_floor=1e-4):
     return x.new_empty(x.shape, dtype=FP8), x.new_empty(x.shape[:-1], dtype=torch.float32)
 
 
-@torch.library.custom_op("hy_nomas_amd::ln_modulate_quantize_fp8", mutates_args=())
-def ln_modulate_quantize_fp8(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
-                             eps: float = 1e-6,
-                             amax_floor: float = 1e-4) -> tuple[torch.Tensor, torch.Tensor]:
+def ln_modulate_quantize_fp8(x, shift, scale, eps: float = 1e-6, amax_floor: float = 1e-4, *,
+                             residual=None):
     """LayerNorm (no affine) + adaLN modulate + per-token e4m3 quantization of a
     bf16 [B, L, C] tensor in one pass: the codes and scales of
     quantize_rows_fp8(modulate(layer_norm(x), shift, scale)) with shift and
     scale bf16 [B, C] (nomas_compile_prepost.py:14-15,40-43,81-84). Returns
-    codes [B*L, C] and fp32 scales [B*L]."""
+    codes [B*L, C] and fp32 scales [B*L].
+
+    With ``residual`` = (y [B, L, C], gate [B, C]) x is first replaced by
+    gated_residual(x, y, gate) in the same pass; returns that x too, before the
+    codes and scales."""
+    if residual is None:
+        return _ln_modulate_quantize_op(x, shift, scale, eps, amax_floor)
+    return _residual_ln_modulate_quantize_op(x, *residual, shift, scale, eps, amax_floor)
+
+
+@torch.library.custom_op("hy_nomas_amd::ln_modulate_quantize_fp8", mutates_args=())
+def _ln_modulate_quantize_op(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
+                             eps: float = 1e-6,
+                             amax_floor: float = 1e-4) -> tuple[torch.Tensor, torch.Tensor]:
     _gpu(x, shift, scale)
     if x.dtype != torch.bfloat16 or shift.dtype != torch.bfloat16 or scale.dtype != torch.bfloat16:
         raise TypeError("ln_modulate_quantize_fp8 expects bf16 tensors")
@@ -86,10 +97,68 @@ def ln_modulate_quantize_fp8(x: torch.Tensor, shift: torch.Tensor, scale: torch.
     return q, s
 
 
-@ln_modulate_quantize_fp8.register_fake
+@_ln_modulate_quantize_op.register_fake
 def _(x, shift, scale, eps=1e-6, amax_floor=1e-4):
     n = x.shape[0] * x.shape[1]
     return x.new_empty((n, x.shape[2]), dtype=FP8), x.new_empty((n,), dtype=torch.float32)
+
+
+def _residual_args(x, y, gate, what: str):
+    """Checks of x and y bf16 [B, L, C] and gate bf16 [B, C]; contiguous x, y and gate."""
+    _gpu(x, y, gate)
+    if x.dtype != torch.bfloat16 or y.dtype != torch.bfloat16 or gate.dtype != torch.bfloat16:
+        raise TypeError(f"{what} expects bf16 tensors")
+    if x.ndim != 3 or y.shape != x.shape or gate.shape != (x.shape[0], x.shape[2]):
+        raise ValueError(f"{what}: x and y [B, L, C] with gate [B, C]")
+    return x.contiguous(), y.contiguous(), gate.contiguous()
+
+
+@torch.library.custom_op("hy_nomas_amd::gated_residual", mutates_args=())
+def gated_residual(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
+    """x + y * gate for bf16 [B, L, C] x and y and a [B, C] gate, with the bf16
+    roundings of the two tensor ops (nomas_compile_prepost.py:87-88)."""
+    x, y, gate = _residual_args(x, y, gate, "gated_residual")
+    B, Lt, C = x.shape
+    out = torch.empty_like(x)
+    with torch.cuda.device(x.device):
+        L.check(L.load().hn_gated_residual(x.data_ptr(), y.data_ptr(), gate.data_ptr(), C, out.data_ptr(),
+                                           B * Lt, C, max(Lt, 1), _stream(x)), "hn_gated_residual")
+    return out
+
+
+@gated_residual.register_fake
+def _(x, y, gate):
+    return x.new_empty(x.shape)
+
+
+@torch.library.custom_op("hy_nomas_amd::residual_ln_modulate_quantize_fp8", mutates_args=())
+def _residual_ln_modulate_quantize_op(
+        x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
+        eps: float = 1e-6, amax_floor: float = 1e-4) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    x, y, gate = _residual_args(x, y, gate, "ln_modulate_quantize_fp8")
+    _gpu(shift, scale)
+    if shift.dtype != torch.bfloat16 or scale.dtype != torch.bfloat16:
+        raise TypeError("ln_modulate_quantize_fp8 expects bf16 tensors")
+    if shift.shape != gate.shape or scale.shape != gate.shape:
+        raise ValueError("ln_modulate_quantize_fp8: gate, shift and scale [B, C]")
+    shift, scale = shift.contiguous(), scale.contiguous()
+    B, Lt, C = x.shape
+    out = torch.empty_like(x)
+    q = torch.empty((B * Lt, C), dtype=FP8, device=x.device)
+    s = torch.empty((B * Lt,), dtype=torch.float32, device=x.device)
+    with torch.cuda.device(x.device):
+        L.check(L.load().hn_residual_ln_mod_quantize_fp8(
+            x.data_ptr(), y.data_ptr(), gate.data_ptr(), C, out.data_ptr(), B * Lt, C, max(Lt, 1),
+            shift.data_ptr(), scale.data_ptr(), C, eps, amax_floor, q.data_ptr(), s.data_ptr(), _stream(x)),
+            "hn_residual_ln_mod_quantize_fp8")
+    return out, q, s
+
+
+@_residual_ln_modulate_quantize_op.register_fake
+def _(x, y, gate, shift, scale, eps=1e-6, amax_floor=1e-4):
+    n = x.shape[0] * x.shape[1]
+    return (x.new_empty(x.shape), x.new_empty((n, x.shape[2]), dtype=FP8),
+            x.new_empty((n,), dtype=torch.float32))
 
 
 @torch.library.custom_op("hy_nomas_amd::quantize_blockwise_fp8", mutates_args=())

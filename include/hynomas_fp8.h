@@ -82,6 +82,19 @@ int hn_ln_mod_quantize_fp8(const void *x, int64_t rows, int64_t cols, int64_t ro
                            const void *shift, const void *scale_mod, int64_t mod_stride, float eps,
                            float amax_floor, void *q, float *scale, void *stream);
 
+/* The block's gated residual out = bf16(x + bf16(y * gate[b])), the bf16 tensor
+ * ops of nomas_compile_prepost.py:78-79,87-88. x, y, out: bf16 [rows, cols]
+ * contiguous (out may be x); gate: bf16 [B, cols] with batch stride gate_stride
+ * (elements), row r using batch r / rows_per_batch. cols % 8 == 0, cols <= 8192. */
+int hn_gated_residual(const void *x, const void *y, const void *gate, int64_t gate_stride, void *out,
+                      int64_t rows, int64_t cols, int64_t rows_per_batch, void *stream);
+
+/* hn_gated_residual into x_out, then hn_ln_mod_quantize_fp8 of it, in one pass. */
+int hn_residual_ln_mod_quantize_fp8(const void *x, const void *y, const void *gate, int64_t gate_stride,
+                                    void *x_out, int64_t rows, int64_t cols, int64_t rows_per_batch,
+                                    const void *shift, const void *scale_mod, int64_t mod_stride,
+                                    float eps, float amax_floor, void *q, float *scale, void *stream);
+
 /* 128x128 blockwise FP8 quantization, rows zero-padded to a multiple of 128.
  * x: bf16 [rows, cols] contiguous; q: e4m3 [rows, cols]; scale: fp32
  * [ceil(rows/128), cols/128]; cols % 128 == 0. Scale rule HN_SCALE_CLAMP with

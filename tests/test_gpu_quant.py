@@ -246,6 +246,27 @@ def test_ln_modulate_quantize_bit_exact(O, dev, B, L, C):
     assert np.array_equal(s.cpu().numpy(), so)
 
 
+@pytest.mark.parametrize("B,L,C", [(1, 300, 3072), (2, 130, 640), (3, 5, 8), (1, 7, 8192), (1, 33, 1032)])
+def test_gated_residual_kernels(dev, B, L, C):
+    """The residual equals the two bf16 tensor ops bit for bit, alone and fused;
+    the fused codes and scales equal ln_modulate_quantize_fp8 of it; widths with
+    whole and partly idle waves; gates as strided parts of a [B, 6 C] vector."""
+    print(f"case gated residual {B}x{L}x{C}", flush=True)
+    ops = pkg_module("ops")
+    x, sh, sc = _ln_inputs(dev, B, L, C, B * L + C)
+    y, parts, _ = _ln_inputs(dev, B, L, 6 * C, 3)
+    y, gate = y[..., :C].contiguous(), parts.chunk(6, dim=-1)[2]
+    ref = x + y * gate.unsqueeze(1)
+    assert torch.equal(ops.gated_residual(x, y, gate), ref)
+    out, q, s = ops.ln_modulate_quantize_fp8(x, sh, sc, 1e-6, residual=(y, gate))
+    qr, sr = ops.ln_modulate_quantize_fp8(ref, sh, sc, 1e-6)
+    assert torch.equal(out, ref) and np.array_equal(u8(q), u8(qr)) and torch.equal(s, sr)
+    with pytest.raises(ValueError):
+        ops.gated_residual(x, y[:, 1:], gate)
+    with pytest.raises(TypeError):
+        ops.gated_residual(x, y.float(), gate)
+
+
 def test_ln_modulate_quantize_matches_unfused_torch_path(dev):
     """Against F.layer_norm + the bf16 modulate ops + quantize_rows_fp8 on the GPU
     (torch's own LayerNorm summation): codes agree except where a LayerNorm output
