@@ -69,6 +69,8 @@ _lock = threading.Lock()
 def load(path: Path | str | None = None) -> ctypes.CDLL:
     """Load (once) and return the library with argtypes set. Raises if absent."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

@@ -5,9 +5,15 @@ launches on the current stream of the input's device, and raises on CPU
 tensors: the FP8 path has no CPU fallback. The custom-op + register_fake
 pattern is the one the reference uses for its FP8 GEMM
 (hymm/models/vae/pixelumm_decoder/cutlass_fp8.py:47-57).
+
+Plain eager inference calls an op's implementation without the dispatcher
+(``eager_op``): the trip through torch's custom-op layers costs more host time
+than a launch, and the small calls are bound by it.
 """
 from __future__ import annotations
 
+import contextlib
+import functools
 import math
 from typing import Optional
 
@@ -25,7 +31,72 @@ def _gpu(*tensors) -> None:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+def _on(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing where it is current already."""
+    return contextlib.nullcontext() if device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
+_TENSOR = (torch.Tensor, torch.nn.Parameter)
+_KINDS = {"Tensor": _TENSOR, "Optional[Tensor]": (*_TENSOR, type(None)), "int": (int,), "float": (float, int),
+          "Optional[float]": (float, int, type(None))}
+
+
+def _observed() -> bool:
+    """Whether something other than the kernel would see a call of an op: a
+    trace, a torch_function or torch_dispatch mode, a functorch transform,
+    forward-mode AD or the autograd profiler."""
+    return bool(torch._C._get_tracing_state() is not None or torch._C._len_torch_function_stack()
+                or torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0 or torch.autograd._profiler_enabled())
+
+
+def eager_op(name: str, mutates_args=()):
+    """``torch.library.custom_op`` whose plain eager calls skip the dispatcher.
+
+    A call goes straight to the implementation when every argument is of
+    exactly its schema's type (plain tensors and numbers, no subclass), no tensor
+    would be recorded by autograd and nothing observes the call (_observed, or
+    torch.compile); every other call goes through the registered op. Mutated
+    tensors get the version bump that the op gives them. Host time of an FP8
+    linear 45 -> 24 us, of a K/V cache write 41 -> 31 us."""
+    def wrap(fn):
+        op = torch.library.custom_op(name, fn, mutates_args=mutates_args)
+        args = op._opoverload._schema.arguments
+        names = [a.name for a in args]
+        kinds = [_KINDS[str(a.type)] for a in args]
+        by_name = dict(zip(names, kinds))
+        required = sum(not a.has_default_value() for a in args)
+        mutated = [(i, n) for i, n in enumerate(names) if n in mutates_args]
+
+        def plain(pos, kw) -> bool:
+            if len(pos) > len(kinds) or (len(pos) < required and any(n not in kw for n in names[len(pos):required])):
+                return False
+            grad = torch.is_grad_enabled()
+            for v, kind in zip(pos, kinds):
+                if type(v) not in kind or (grad and isinstance(v, torch.Tensor) and v.requires_grad):
+                    return False
+            for n, v in kw.items():
+                if type(v) not in by_name.get(n, ()) or (grad and isinstance(v, torch.Tensor) and v.requires_grad):
+                    return False
+            return not _observed()
+
+        @functools.wraps(fn)
+        def call(*pos, **kw):
+            if torch.compiler.is_compiling() or not plain(pos, kw):
+                return op(*pos, **kw)
+            out = fn(*pos, **kw)
+            if mutated:
+                seen = [pos[i] if i < len(pos) else kw.get(n) for i, n in mutated]
+                torch.autograd.graph.increment_version([t for t in seen if t is not None and not t.is_inference()])
+            return out
+
+        call.register_fake = op.register_fake
+        call.impl = fn
+        return call
+    return wrap
 
 
 def _bytes(t: torch.Tensor) -> torch.Tensor:
@@ -35,23 +106,29 @@ def _bytes(t: torch.Tensor) -> torch.Tensor:
 # --------------------------------------------------------------------------
 # quantizers
 
-@torch.library.custom_op("hy_nomas_amd::quantize_rows_fp8", mutates_args=())
+@eager_op("hy_nomas_amd::quantize_rows_fp8", mutates_args=())
 def quantize_rows_fp8(x: torch.Tensor, scale_mode: int = L.HN_SCALE_CLAMP,
                       amax_floor: float = 1e-4) -> tuple[torch.Tensor, torch.Tensor]:
     """Per-row e4m3 codes and fp32 scales of a bf16 [..., C] tensor."""
     _gpu(x)
     if x.dtype != torch.bfloat16:
         raise TypeError("quantize_rows_fp8 expects bf16 input")
-    x2 = x.reshape(-1, x.shape[-1])
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
-    q = torch.empty(x2.shape, dtype=FP8, device=x.device)
-    s = torch.empty((x2.shape[0],), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    q, s = _quantize_matrix(x if x.ndim == 2 else x.reshape(-1, x.shape[-1]), scale_mode, amax_floor)
+    return (q, s) if x.ndim == 2 else (q.view(x.shape), s.view(x.shape[:-1]))
+
+
+def _quantize_matrix(x, scale_mode: int, amax_floor: float):
+    if x.stride(-1) != 1:
+        x = x.contiguous()
+    rows, cols = x.shape
+    device = x.device
+    q = torch.empty((rows, cols), dtype=FP8, device=device)
+    s = torch.empty((rows,), dtype=torch.float32, device=device)
+    with _on(device):
         L.check(L.load().hn_quantize_rows_fp8(
-            x2.data_ptr(), x2.shape[0], x2.shape[1], x2.stride(0), scale_mode, amax_floor,
+            x.data_ptr(), rows, cols, x.stride(0), scale_mode, amax_floor,
             q.data_ptr(), s.data_ptr(), _stream(x)), "hn_quantize_rows_fp8")
-    return q.view(x.shape), s.view(x.shape[:-1])
+    return q, s
 
 
 @quantize_rows_fp8.register_fake
@@ -75,7 +152,7 @@ def ln_modulate_quantize_fp8(x, shift, scale, eps: float = 1e-6, amax_floor: flo
     return _residual_ln_modulate_quantize_op(x, *residual, shift, scale, eps, amax_floor)
 
 
-@torch.library.custom_op("hy_nomas_amd::ln_modulate_quantize_fp8", mutates_args=())
+@eager_op("hy_nomas_amd::ln_modulate_quantize_fp8", mutates_args=())
 def _ln_modulate_quantize_op(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
                              eps: float = 1e-6,
                              amax_floor: float = 1e-4) -> tuple[torch.Tensor, torch.Tensor]:
@@ -90,7 +167,7 @@ def _ln_modulate_quantize_op(x: torch.Tensor, shift: torch.Tensor, scale: torch.
     B, Lt, C = x.shape
     q = torch.empty((B * Lt, C), dtype=FP8, device=x.device)
     s = torch.empty((B * Lt,), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         L.check(L.load().hn_ln_mod_quantize_fp8(
             x.data_ptr(), B * Lt, C, max(Lt, 1), shift.data_ptr(), scale.data_ptr(), C, eps,
             amax_floor, q.data_ptr(), s.data_ptr(), _stream(x)), "hn_ln_mod_quantize_fp8")
@@ -113,14 +190,14 @@ def _residual_args(x, y, gate, what: str):
     return x.contiguous(), y.contiguous(), gate.contiguous()
 
 
-@torch.library.custom_op("hy_nomas_amd::gated_residual", mutates_args=())
+@eager_op("hy_nomas_amd::gated_residual", mutates_args=())
 def gated_residual(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """x + y * gate for bf16 [B, L, C] x and y and a [B, C] gate, with the bf16
     roundings of the two tensor ops (nomas_compile_prepost.py:87-88)."""
     x, y, gate = _residual_args(x, y, gate, "gated_residual")
     B, Lt, C = x.shape
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         L.check(L.load().hn_gated_residual(x.data_ptr(), y.data_ptr(), gate.data_ptr(), C, out.data_ptr(),
                                            B * Lt, C, max(Lt, 1), _stream(x)), "hn_gated_residual")
     return out
@@ -131,7 +208,7 @@ def _(x, y, gate):
     return x.new_empty(x.shape)
 
 
-@torch.library.custom_op("hy_nomas_amd::residual_ln_modulate_quantize_fp8", mutates_args=())
+@eager_op("hy_nomas_amd::residual_ln_modulate_quantize_fp8", mutates_args=())
 def _residual_ln_modulate_quantize_op(
         x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor,
         eps: float = 1e-6, amax_floor: float = 1e-4) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -146,7 +223,7 @@ def _residual_ln_modulate_quantize_op(
     out = torch.empty_like(x)
     q = torch.empty((B * Lt, C), dtype=FP8, device=x.device)
     s = torch.empty((B * Lt,), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         L.check(L.load().hn_residual_ln_mod_quantize_fp8(
             x.data_ptr(), y.data_ptr(), gate.data_ptr(), C, out.data_ptr(), B * Lt, C, max(Lt, 1),
             shift.data_ptr(), scale.data_ptr(), C, eps, amax_floor, q.data_ptr(), s.data_ptr(), _stream(x)),
@@ -161,7 +238,7 @@ def _(x, y, gate, shift, scale, eps=1e-6, amax_floor=1e-4):
             x.new_empty((n,), dtype=torch.float32))
 
 
-@torch.library.custom_op("hy_nomas_amd::quantize_blockwise_fp8", mutates_args=())
+@eager_op("hy_nomas_amd::quantize_blockwise_fp8", mutates_args=())
 def quantize_blockwise_fp8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """128x128 blockwise e4m3 codes [M,K] and scales [ceil(M/128), K/128]."""
     _gpu(x)
@@ -171,7 +248,7 @@ def quantize_blockwise_fp8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]
     m, k = x.shape
     q = torch.empty((m, k), dtype=FP8, device=x.device)
     s = torch.empty(((m + 127) // 128, k // 128), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         L.check(L.load().hn_quantize_blockwise_fp8(x.data_ptr(), m, k, q.data_ptr(), s.data_ptr(),
                                                    _stream(x)), "hn_quantize_blockwise_fp8")
     return q, s
@@ -187,7 +264,7 @@ def _(x):
 # --------------------------------------------------------------------------
 # GEMMs
 
-@torch.library.custom_op("hy_nomas_amd::gemm_fp8_rowcol", mutates_args=())
+@eager_op("hy_nomas_amd::gemm_fp8_rowcol", mutates_args=())
 def gemm_fp8_rowcol(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torch.Tensor,
                     bias: Optional[torch.Tensor] = None, act: int = L.HN_ACT_NONE) -> torch.Tensor:
     """act(a b^T * sa[m] * sb[n] + bias[n]) in bf16; a e4m3 [M,K], b e4m3 [N,K]."""
@@ -205,7 +282,7 @@ def gemm_fp8_rowcol(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor, sb: torc
     if b.shape[1] != k or sa.numel() != m or sb.numel() != n or (bias is not None and bias.numel() != n):
         raise ValueError("gemm_fp8_rowcol shape mismatch")
     out = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
-    with torch.cuda.device(a.device):
+    with _on(a.device):
         L.check(L.load().hn_gemm_fp8_rowcol(
             a.data_ptr(), b.data_ptr(), sa.contiguous().data_ptr(), sb.contiguous().data_ptr(),
             None if bias is None else bias.contiguous().data_ptr(), out.data_ptr(),
@@ -218,7 +295,7 @@ def _(a, b, sa, sb, bias=None, act=L.HN_ACT_NONE):
     return a.new_empty((a.shape[0], b.shape[0]), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("hy_nomas_amd::gemm_fp8_blockwise", mutates_args=())
+@eager_op("hy_nomas_amd::gemm_fp8_blockwise", mutates_args=())
 def gemm_fp8_blockwise(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor,
                        sb: torch.Tensor) -> torch.Tensor:
     """The reference extension's gemm(a, b, sa, sb) with 128x128 block scales."""
@@ -241,7 +318,7 @@ def gemm_fp8_blockwise(a: torch.Tensor, b: torch.Tensor, sa: torch.Tensor,
     if sb.dim() != 2 or tuple(sb.shape) != (n // 128, k // 128):
         raise RuntimeError("Invalid weight scales")
     out = torch.empty((m, n), dtype=torch.bfloat16, device=a.device)
-    with torch.cuda.device(a.device):
+    with _on(a.device):
         L.check(L.load().hn_gemm_fp8_blockwise(a.data_ptr(), b.data_ptr(), sa.data_ptr(),
                                                sb.data_ptr(), out.data_ptr(), m, n, k,
                                                _stream(a)), "hn_gemm_fp8_blockwise")
@@ -253,13 +330,19 @@ def _(a, b, sa, sb):
     return a.new_empty((a.shape[0], b.shape[0]), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("hy_nomas_amd::linear_fp8", mutates_args=())
+@eager_op("hy_nomas_amd::linear_fp8", mutates_args=())
 def linear_fp8(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
                bias: Optional[torch.Tensor] = None, act: int = L.HN_ACT_NONE) -> torch.Tensor:
     """Per-token dynamic e4m3 activation quant + per-channel-scaled FP8 GEMM.
     x bf16 [M, K] -> bf16 [M, N]."""
-    qx, sx = quantize_rows_fp8(x, L.HN_SCALE_CLAMP, 1e-4)
-    return gemm_fp8_rowcol(qx, weight, sx, weight_scale, bias, act)
+    if x.ndim != 2:
+        qx, sx = quantize_rows_fp8.impl(x, L.HN_SCALE_CLAMP, 1e-4)
+    else:
+        _gpu(x)
+        if x.dtype != torch.bfloat16:
+            raise TypeError("quantize_rows_fp8 expects bf16 input")
+        qx, sx = _quantize_matrix(x, L.HN_SCALE_CLAMP, 1e-4)
+    return gemm_fp8_rowcol.impl(qx, weight, sx, weight_scale, bias, act)
 
 
 @linear_fp8.register_fake
@@ -320,7 +403,7 @@ def kv_quantize_(codes, scale, x, start: int, status=None) -> None:
     _kv_quantize_op(codes, scale, x, start, status)
 
 
-@torch.library.custom_op("hy_nomas_amd::kv_quantize_pair_",
+@eager_op("hy_nomas_amd::kv_quantize_pair_",
                          mutates_args=("k_codes", "v_codes", "k_scale", "v_scale", "status"))
 def _kv_quantize_pair_op(k_codes: torch.Tensor, v_codes: torch.Tensor, k_scale: torch.Tensor,
                          v_scale: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -340,7 +423,7 @@ def _kv_quantize_pair_op(k_codes: torch.Tensor, v_codes: torch.Tensor, k_scale: 
     sp = _status_ptr(status)
     _gpu(k_codes, v_codes, k_scale, v_scale, k, v, status)
     B, Lt, H, D = k.shape
-    with torch.cuda.device(k.device):
+    with _on(k.device):
         L.check(L.load().hn_kv_quantize_pair(
             fmt, k.data_ptr(), v.data_ptr(), L.strides(k), B, Lt, H, D,
             k_codes.data_ptr(), v_codes.data_ptr(), L.strides(k_codes),
@@ -353,7 +436,7 @@ def _(k_codes, v_codes, k_scale, v_scale, k, v, start, status):
     return None
 
 
-@torch.library.custom_op("hy_nomas_amd::kv_quantize_", mutates_args=("codes", "scale", "status"))
+@eager_op("hy_nomas_amd::kv_quantize_", mutates_args=("codes", "scale", "status"))
 def _kv_quantize_op(codes: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, start: int,
                     status: Optional[torch.Tensor]) -> None:
     """Quantize bf16 values [B,L,H,D] into one cache tensor at ``start``
@@ -363,7 +446,7 @@ def _kv_quantize_op(codes: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, s
     sp = _status_ptr(status)
     _gpu(codes, scale, x, status)
     B, Lt, H, D = x.shape
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         L.check(L.load().hn_kv_quantize(
             fmt, x.data_ptr(), L.strides(x), B, Lt, H, D, codes.data_ptr(), L.strides(codes),
             scale.data_ptr(), L.strides(scale), cap, start, sp, _stream(x)), "hn_kv_quantize")
@@ -374,7 +457,7 @@ def _(codes, scale, x, start, status):
     return None
 
 
-@torch.library.custom_op("hy_nomas_amd::kv_dequantize", mutates_args=())
+@eager_op("hy_nomas_amd::kv_dequantize", mutates_args=())
 def kv_dequantize(codes: torch.Tensor, scale: torch.Tensor, valid_len: int) -> torch.Tensor:
     """bf16(code * scale) for tokens [0, valid_len): a new [B, valid_len, H, D] tensor."""
     _gpu(codes, scale)
@@ -383,7 +466,7 @@ def kv_dequantize(codes: torch.Tensor, scale: torch.Tensor, valid_len: int) -> t
     y = torch.empty((B, valid_len, H, D), dtype=torch.bfloat16, device=codes.device)
     if valid_len == 0:
         return y
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         L.check(L.load().hn_kv_dequantize(
             fmt, codes.data_ptr(), L.strides(codes), scale.data_ptr(), L.strides(scale),
             B, valid_len, H, D, y.data_ptr(), L.strides(y), _stream(codes)), "hn_kv_dequantize")
@@ -425,14 +508,14 @@ def _qk_launch(q, k, v, q_weight, k_weight, cos, sin, eps, cache, start, status=
         fmt = L.HN_KV_FP8
         cargs = (None, None, None, None, None, None, 0, start, None)
     _gpu(q, k, v, q_weight, k_weight, cos, sin, status, *(cache or ()))
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         L.check(L.load().hn_qk_norm_rope_kv(
             fmt, q.data_ptr(), k.data_ptr(), v.data_ptr(), L.strides(q), B, Lt, H, D,
             qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(), cos.stride(0), eps,
             *cargs, _stream(q)), "hn_qk_norm_rope_kv")
 
 
-@torch.library.custom_op("hy_nomas_amd::qk_norm_rope_", mutates_args=("q", "k"))
+@eager_op("hy_nomas_amd::qk_norm_rope_", mutates_args=("q", "k"))
 def qk_norm_rope_(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_weight: torch.Tensor,
                   k_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, eps: float) -> None:
     """In place: q, k <- RoPE(RMSNorm(q)), RoPE(RMSNorm(k)) for bf16 [B, L, H, 128]
@@ -455,7 +538,7 @@ def qk_norm_rope_kv_(q, k, v, q_weight, k_weight, cos, sin, eps: float, k_codes,
                         start, status)
 
 
-@torch.library.custom_op("hy_nomas_amd::qk_norm_rope_kv_",
+@eager_op("hy_nomas_amd::qk_norm_rope_kv_",
                          mutates_args=("q", "k", "k_codes", "v_codes", "k_scale", "v_scale", "status"))
 def _qk_norm_rope_kv_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_weight: torch.Tensor,
                         k_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, eps: float,
@@ -488,7 +571,7 @@ def _valid_bytes(mask: Optional[torch.Tensor], rows: int, cols: int, what: str):
     return mask.view(torch.uint8), stride
 
 
-@torch.library.custom_op("hy_nomas_amd::attn_fp8kv", mutates_args=())
+@eager_op("hy_nomas_amd::attn_fp8kv", mutates_args=())
 def attn_fp8kv(q: torch.Tensor, k_codes: torch.Tensor, v_codes: torch.Tensor,
                k_scale: torch.Tensor, v_scale: torch.Tensor, kv_len: int,
                k_cur: Optional[torch.Tensor] = None, v_cur: Optional[torch.Tensor] = None,
@@ -537,7 +620,7 @@ def attn_fp8kv(q: torch.Tensor, k_codes: torch.Tensor, v_codes: torch.Tensor,
     uvb, uvs = _valid_bytes(cur_valid if cur_len else None, B, cur_len, "cur_valid")
     _gpu(q, k_codes, v_codes, k_scale, v_scale, k_cur, v_cur, kvb, uvb)
     out = torch.empty((B, Lq, H, D), dtype=torch.bfloat16, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         lib = L.load()
         ws_bytes = lib.hn_attn_fp8kv_workspace_size(B, Lq, H, D, kv_len, cur_len)
         ws = torch.empty((ws_bytes,), dtype=torch.uint8, device=q.device) if ws_bytes else None

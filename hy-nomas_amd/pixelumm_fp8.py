@@ -66,7 +66,7 @@ def quantize_blockwise(x: torch.Tensor):
 _quantize_blockwise = quantize_blockwise
 
 
-@torch.library.custom_op("hy_nomas_amd::blockwise_linear", mutates_args=())
+@ops.eager_op("hy_nomas_amd::blockwise_linear")
 def _linear(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
     codes, x_scale = quantize_blockwise(x)
     y = load_extension().gemm(codes, weight, x_scale, scale)

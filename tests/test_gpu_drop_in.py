@@ -168,3 +168,45 @@ def test_enable_fp8_on_a_stand_in_decoder(O, dev):
     assert after[(21, 512, 256)] == before.get((21, 512, 256), 0) + 1
     with pytest.raises(RuntimeError, match="inference"):
         model[0](x)   # grad enabled
+
+
+def test_eager_calls_past_the_dispatcher_are_the_registered_ops(dev):
+    """Plain eager calls run the implementation directly; modes, profilers,
+    autograd inputs, subclasses and schema errors still meet the registered op,
+    and a mutated cache gets the op's version bump."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    ops, kvc = pkg_module("ops"), pkg_module("fp8_kv_cache")
+    g = torch.Generator(device=dev).manual_seed(1)
+    x = torch.randn(40, 256, device=dev, generator=g).to(torch.bfloat16)
+    w, s = ops.quantize_rows_fp8(torch.randn(384, 256, device=dev, generator=g).to(torch.bfloat16))
+    y = ops.linear_fp8(x, w, s)
+    assert torch.equal(y, torch.ops.hy_nomas_amd.linear_fp8(x, w, s, None, 0))
+
+    seen = []
+
+    class Record(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Record():
+        assert torch.equal(ops.linear_fp8(x, w, s), y)
+    assert any("linear_fp8" in f for f in seen), seen
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        ops.linear_fp8(x, w, s)
+    assert any("hy_nomas_amd::linear_fp8" in e.key for e in prof.key_averages())
+    assert ops.linear_fp8(x.clone().requires_grad_(), w, s).requires_grad  # the op's own autograd kernel
+    with torch.no_grad():
+        assert not ops.linear_fp8(x.clone().requires_grad_(), w, s).requires_grad
+    with pytest.raises(RuntimeError):
+        ops.linear_fp8(x, w, s, None, 0.5)                       # act: int in the schema
+    cache = kvc.make_fp8_kv_block(1, 64, 2, 128, device=dev)
+    kv = torch.randn(1, 8, 2, 128, device=dev, generator=g).to(torch.bfloat16)
+    before = {n: t._version for n, t in cache.items()}
+    kvc.quantize_kv_pair_into(cache, kv, kv, 0, status=torch.zeros(1, dtype=torch.int32, device=dev))
+    assert all(cache[n]._version == before[n] + 1 for n in cache)
+    with torch.inference_mode():
+        assert torch.equal(ops.linear_fp8(x, w, s), y)
+        icache = kvc.make_fp8_kv_block(1, 64, 2, 128, device=dev)
+        kvc.quantize_kv_pair_into(icache, kv, kv, 0)
+        assert torch.equal(icache["k_scale"][:, :8], cache["k_scale"][:, :8])
