@@ -170,8 +170,7 @@ def causal_attention_with_cache_mp(q, k, v, kv_cache, cache_valid_len: int = 0,
     B = img_q.shape[0]
     img_len, txt_len = img_k.shape[1], txt_k.shape[1]
     dev = img_k.device
-    cur_k = torch.cat([img_k, txt_k], dim=1)
-    cur_v = torch.cat([img_v, txt_v], dim=1)
+    q_full, cur_k, cur_v = ops.join_tokens(img_q, txt_q, img_k, txt_k, img_v, txt_v)
     cache_k, cache_v = (cur_k, cur_v) if cache_txt else (img_k, img_v)
 
     # One canonical history slot may serve the B current (CFG) branches, read
@@ -217,7 +216,6 @@ def causal_attention_with_cache_mp(q, k, v, kv_cache, cache_valid_len: int = 0,
     else:
         tail_k, tail_v, tail_valid = img_k, img_v, None
 
-    q_full = torch.cat([img_q, txt_q], dim=1)
     with stage("cache_attention"):
         hidden = chunk_attention(q_full, kv_cache, cache_valid_len, k_cur=tail_k.contiguous(),
                                  v_cur=tail_v.contiguous(), cache_valid=history_valid,

@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void quantize_rows_wide_kernel(
 // stride mod_stride).
 //
 // RES: x is first the block's gated residual, x <- bf16(x + bf16(y * gate[b]))
-// (bf16 tensor ops of nomas_compile_prepost.py:78-79), written to `out`. As
+// (bf16 tensor ops of nomas_compile_prepost.py:75-88), written to `out`. As
 // separate kernels the product, the sum and the LayerNorm read or write 8 bf16
 // rows and one row of codes; here 3 and one: 10800 x 3072 89 -> 58 us.
 struct Residual {
@@ -288,6 +288,49 @@ __global__ __launch_bounds__(256) void ln_mod_quantize_kernel(
                 if (FULL || c < nchunks) *reinterpret_cast<uint2*>(qr + (int64_t)c * 8) = encode8<decltype(form)::value>(v[i], d);
             }
         });
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Up to three token concatenations out[i] = [a[i] | b[i]] along dim 1 of [B, L, H,
+// 128] bf16 tensors (a stream pair's Q, K and V before the cached attention), in
+// one launch: 16 lanes move a (token, head) row of 256 bytes, 4 rows in flight
+// per lane. HBM bound; 10800 + 256 tokens x 24 heads, three tensors of QKV views:
+// 267 us as tensor concatenations (1.5 TB/s) -> 84 us.
+struct JoinArgs {
+    const uint16_t* src[3][2];
+    int64_t st[3][2][3];  // [tensor][part][batch, token, head], elements
+    uint16_t* out[3];
+    int64_t rows;         // B (L0 + L1) H
+    int64_t L0, L;
+    int H;
+};
+
+__global__ __launch_bounds__(256) void join_tokens_kernel(JoinArgs a) {
+    const int n = blockIdx.y, lane16 = threadIdx.x & 15, g = threadIdx.x >> 4;
+    const int64_t per_batch = a.L * a.H;
+    for (int64_t r0 = (int64_t)blockIdx.x * 64; r0 < a.rows; r0 += (int64_t)gridDim.x * 64) {
+        const int64_t b0 = r0 / per_batch;
+        uint4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t row = r0 + 16 * k + g < a.rows ? r0 + 16 * k + g : a.rows - 1;
+            int64_t b = b0, in = row - b0 * per_batch;
+            while (in >= per_batch) {  // a unit may cross into the next batches
+                in -= per_batch;
+                ++b;
+            }
+            const uint32_t t = (uint32_t)in / (uint32_t)a.H, h = (uint32_t)in - t * (uint32_t)a.H;
+            const int part = t >= (uint32_t)a.L0;
+            const int64_t tt = part ? t - a.L0 : t;
+            v[k] = *reinterpret_cast<const uint4*>(a.src[n][part] + b * a.st[n][part][0] + tt * a.st[n][part][1] +
+                                                   h * a.st[n][part][2] + lane16 * 8);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t row = r0 + 16 * k + g;
+            if (row < a.rows) *reinterpret_cast<uint4*>(a.out[n] + row * 128 + lane16 * 8) = v[k];
+        }
     }
 }
 
@@ -864,4 +907,38 @@ extern "C" int hn_e4m3_encode_range(uint32_t first, int64_t n, void* out, void* 
     e4m3_encode_range_kernel<<<(unsigned)grid, 256, 0, (hipStream_t)stream>>>(first, words,
                                                                               (uint32_t*)out);
     return check_launch("hn_e4m3_encode_range");
+}
+
+extern "C" int hn_join_tokens(int n, const void* const* a, const int64_t* as, const void* const* b,
+                              const int64_t* bs, int64_t B, int64_t La, int64_t Lb, int64_t H, int64_t D,
+                              void* const* out, void* stream) {
+    HN_REQUIRE(n >= 1 && n <= 3 && a && as && b && bs && out, HN_E_ARG, "hn_join_tokens: 1 to 3 tensor pairs");
+    HN_REQUIRE(D == 128 && B >= 0 && La >= 0 && Lb >= 0 && H > 0, HN_E_ARG, "hn_join_tokens: invalid shape");
+    HN_REQUIRE((La + Lb) * H < 0x7fffffffLL, HN_E_ARG, "hn_join_tokens: too many rows per batch");
+    JoinArgs j{};
+    for (int i = 0; i < n; ++i) {
+        const void* const src[2] = {a[i], b[i]};
+        const int64_t* const st[2] = {as + 4 * i, bs + 4 * i};
+        const int64_t len[2] = {La, Lb};
+        for (int k = 0; k < 2; ++k) {
+            j.src[i][k] = (const uint16_t*)src[k];
+            HN_REQUIRE(len[k] == 0 || (src[k] && aligned(src[k], 16)), HN_E_ARG,
+                       "hn_join_tokens: null or misaligned source");
+            HN_REQUIRE(st[k][3] == 1, HN_E_ARG, "hn_join_tokens: the head dim must be contiguous");
+            for (int d = 0; d < 3; ++d) {
+                HN_REQUIRE(st[k][d] % 8 == 0, HN_E_ARG, "hn_join_tokens: strides must be multiples of 8 elements");
+                j.st[i][k][d] = st[k][d];
+            }
+        }
+        HN_REQUIRE(aligned(out[i], 16), HN_E_ARG, "hn_join_tokens: misaligned output");
+        j.out[i] = (uint16_t*)out[i];
+    }
+    j.L0 = La; j.L = La + Lb; j.H = (int)H;
+    j.rows = B * j.L * H;
+    if (j.rows == 0) return HN_OK;
+    for (int i = 0; i < n; ++i) HN_REQUIRE(out[i], HN_E_ARG, "hn_join_tokens: null output");
+    if (const int rc = require_gfx950("hn_join_tokens"); rc != HN_OK) return rc;
+    const dim3 grid((unsigned)stream_grid((j.rows + 63) / 64, 16 / n), (unsigned)n);
+    join_tokens_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(j);
+    return check_launch("hn_join_tokens");
 }

@@ -13,6 +13,7 @@ than a launch, and the small calls are bound by it.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import functools
 import math
 from typing import Optional
@@ -193,7 +194,7 @@ def _residual_args(x, y, gate, what: str):
 @eager_op("hy_nomas_amd::gated_residual", mutates_args=())
 def gated_residual(x: torch.Tensor, y: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     """x + y * gate for bf16 [B, L, C] x and y and a [B, C] gate, with the bf16
-    roundings of the two tensor ops (nomas_compile_prepost.py:87-88)."""
+    roundings of the two tensor ops (nomas_compile_prepost.py:75-88)."""
     x, y, gate = _residual_args(x, y, gate, "gated_residual")
     B, Lt, C = x.shape
     out = torch.empty_like(x)
@@ -555,6 +556,48 @@ def _(q, k, v, q_weight, k_weight, cos, sin, eps, k_codes, v_codes, k_scale, v_s
 
 # --------------------------------------------------------------------------
 # attention
+
+def _joinable(t: torch.Tensor) -> bool:
+    return (t.dtype == torch.bfloat16 and t.ndim == 4 and t.shape[3] == 128 and t.stride(3) == 1
+            and all(s % 8 == 0 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0)
+
+
+def join_tokens(qa, qb, ka, kb, va, vb):
+    """torch.cat([a, b], dim=1) of the q, k and v of two token streams, bf16 [B, L,
+    H, 128] each, in one kernel where it reads their layout."""
+    pairs = (qa, qb, ka, kb, va, vb)
+    if (all(t.is_cuda and t.device == qa.device and _joinable(t) for t in pairs)
+            and all(t.shape == qa.shape for t in (ka, va)) and all(t.shape == qb.shape for t in (kb, vb))
+            and (qa.shape[0], qa.shape[2]) == (qb.shape[0], qb.shape[2])):
+        return _join_tokens_op(*pairs)
+    return torch.cat([qa, qb], dim=1), torch.cat([ka, kb], dim=1), torch.cat([va, vb], dim=1)
+
+
+@eager_op("hy_nomas_amd::join_tokens")
+def _join_tokens_op(qa: torch.Tensor, qb: torch.Tensor, ka: torch.Tensor, kb: torch.Tensor, va: torch.Tensor,
+                    vb: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    B, La, H, D = qa.shape
+    Lb = qb.shape[1]
+    out = tuple(torch.empty((B, La + Lb, H, D), dtype=torch.bfloat16, device=qa.device) for _ in range(3))
+
+    def pointers(ts):
+        return (ctypes.c_void_p * 3)(*(t.data_ptr() for t in ts))
+
+    def strides(ts):
+        return (ctypes.c_int64 * 12)(*(s for t in ts for s in t.stride()))
+
+    a, b = (qa, ka, va), (qb, kb, vb)
+    with _on(qa.device):
+        L.check(L.load().hn_join_tokens(3, pointers(a), strides(a), pointers(b), strides(b), B, La, Lb, H, D,
+                                        pointers(out), _stream(qa)), "hn_join_tokens")
+    return out
+
+
+@_join_tokens_op.register_fake
+def _(qa, qb, ka, kb, va, vb):
+    shape = (qa.shape[0], qa.shape[1] + qb.shape[1], *qa.shape[2:])
+    return qa.new_empty(shape), qa.new_empty(shape), qa.new_empty(shape)
+
 
 def _valid_bytes(mask: Optional[torch.Tensor], rows: int, cols: int, what: str):
     """A key-validity mask as (uint8 view, batch stride): bool or uint8 [rows or

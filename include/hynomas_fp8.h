@@ -83,7 +83,7 @@ int hn_ln_mod_quantize_fp8(const void *x, int64_t rows, int64_t cols, int64_t ro
                            float amax_floor, void *q, float *scale, void *stream);
 
 /* The block's gated residual out = bf16(x + bf16(y * gate[b])), the bf16 tensor
- * ops of nomas_compile_prepost.py:78-79,87-88. x, y, out: bf16 [rows, cols]
+ * ops of nomas_compile_prepost.py:75-88. x, y, out: bf16 [rows, cols]
  * contiguous (out may be x); gate: bf16 [B, cols] with batch stride gate_stride
  * (elements), row r using batch r / rows_per_batch. cols % 8 == 0, cols <= 8192. */
 int hn_gated_residual(const void *x, const void *y, const void *gate, int64_t gate_stride, void *out,
@@ -94,6 +94,15 @@ int hn_residual_ln_mod_quantize_fp8(const void *x, const void *y, const void *ga
                                     void *x_out, int64_t rows, int64_t cols, int64_t rows_per_batch,
                                     const void *shift, const void *scale_mod, int64_t mod_stride,
                                     float eps, float amax_floor, void *q, float *scale, void *stream);
+
+/* n (1 to 3) token concatenations out[i] = [a[i] | b[i]] along dim 1 of bf16 [B, La,
+ * H, 128] and [B, Lb, H, 128] tensors: the q, k, v of the image and text streams
+ * before the cached attention (nomas_cpt.py:614-625). as / bs: n x 4 element
+ * strides (head dim contiguous, the others multiples of 8); out[i]: contiguous
+ * [B, La + Lb, H, 128]. */
+int hn_join_tokens(int n, const void *const *a, const int64_t *as, const void *const *b,
+                   const int64_t *bs, int64_t B, int64_t La, int64_t Lb, int64_t H, int64_t D,
+                   void *const *out, void *stream);
 
 /* 128x128 blockwise FP8 quantization, rows zero-padded to a multiple of 128.
  * x: bf16 [rows, cols] contiguous; q: e4m3 [rows, cols]; scale: fp32

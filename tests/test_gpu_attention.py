@@ -784,3 +784,24 @@ def test_attention_writes_nothing_outside_out(dev, B, H, Lq, n_chunks, chunk, cu
         torch.cuda.current_stream().cuda_stream), "hn_attn_fp8kv")
     assert torch.equal(out, ref)
     assert bool((buf[:, Lq:] == 5.0).all()) and bool((buf[:, :, H:] == 5.0).all())
+
+
+@pytest.mark.parametrize("B,La,Lb,H", [(1, 300, 77, 24), (2, 5, 3, 3), (3, 1, 1, 2), (1, 40, 0, 5), (2, 0, 9, 4)])
+def test_join_tokens_is_torch_cat(dev, B, La, Lb, H):
+    """Contiguous, QKV-strided and [B, H, L, D] sources, units that cross batches,
+    empty parts; layouts the kernel does not read are concatenated by torch."""
+    print(f"case join {B}x({La}+{Lb})x{H}", flush=True)
+    ops = pkg_module("ops")
+    g = torch.Generator(device=dev).manual_seed(La + 10 * Lb)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=dev, generator=g).to(torch.bfloat16)
+
+    qkv = rand(B, La, 3, H, 128)
+    a = (qkv.select(2, 0), rand(B, H, La, 128).transpose(1, 2), qkv.select(2, 2))
+    b = (rand(B, Lb, H, 128), rand(B, Lb, H, 128), rand(B, H, Lb, 128).transpose(1, 2))
+    odd = (rand(B, Lb, H, 130)[..., :128], b[1], b[2])   # a stride of 130 elements
+    for second in (b, odd):
+        got = ops.join_tokens(a[0], second[0], a[1], second[1], a[2], second[2])
+        for x, y, z in zip(got, a, second):
+            assert torch.equal(x, torch.cat([y, z], dim=1))
