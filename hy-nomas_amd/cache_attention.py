@@ -31,7 +31,7 @@ from typing import Optional
 import torch
 
 from . import ops
-from .fp8_kv_cache import is_fp8_kv_cache, is_quantized_kv_cache, quantize_kv_pair_into
+from .fp8_kv_cache import is_fp8_kv_cache, is_quantized_kv_cache, quantize_kv_pair_into, read_flag_later
 from .metrics import stage
 
 
@@ -196,12 +196,12 @@ def causal_attention_with_cache_mp(q, k, v, kv_cache, cache_valid_len: int = 0,
 
     if update_cache:
         new_end = cache_valid_len + cache_k.shape[1]
-        quantize_kv_pair_into(kv_cache, cache_k.detach(), cache_v.detach(), cache_valid_len)
-        if cache_mask is not None:
-            write_mask = torch.ones(B, cache_k.shape[1], dtype=torch.bool, device=dev)
-            if cache_txt and txt_valid is not None:
-                write_mask[:, img_len:] = txt_valid
-            cache_mask[:, cache_valid_len:new_end] = write_mask
+        # The write is validated on the device, and its verdict read once the
+        # attention is enqueued (which reads neither the written tokens nor
+        # their part of cache_mask).
+        flag = torch.empty(1, dtype=torch.int32, device=dev)
+        quantize_kv_pair_into(kv_cache, cache_k.detach(), cache_v.detach(), cache_valid_len, status=flag)
+        refused = read_flag_later(flag) if cache_k.shape[1] else None
 
     # Keys after the history: the current chunk's bf16 K/V (the reference keeps
     # them unquantized for their own attention, nomas_cpt.py:614-625).
@@ -220,6 +220,13 @@ def causal_attention_with_cache_mp(q, k, v, kv_cache, cache_valid_len: int = 0,
         hidden = chunk_attention(q_full, kv_cache, cache_valid_len, k_cur=tail_k.contiguous(),
                                  v_cur=tail_v.contiguous(), cache_valid=history_valid,
                                  cur_valid=tail_valid)
+    if update_cache:
+        if refused is not None:
+            refused()  # ValueError: nothing was written
+        if cache_mask is not None:
+            cache_mask[:, cache_valid_len:new_end] = True
+            if cache_txt and txt_valid is not None:
+                cache_mask[:, cache_valid_len + img_len:new_end] = txt_valid
     if note_dense is not None:
         note_dense()
     img_attn = hidden[:, :img_len].to(img_dtype)

@@ -98,6 +98,23 @@ def _raise_if_flagged(status: torch.Tensor) -> None:
         raise ValueError(_NONFINITE)
 
 
+def read_flag_later(status: torch.Tensor):
+    """Starts reading a write's status word now, in stream order, and returns a
+    function that waits for the read alone and raises ValueError if the write
+    was refused. Work enqueued in between keeps the GPU busy: waiting for the
+    word at once drains the stream, and the host then enqueues behind an idle
+    GPU (about 170 us in a block's write pass)."""
+    word = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    word.copy_(status[:1], non_blocking=True)
+    done = torch.cuda.Event()
+    done.record(torch.cuda.current_stream(status.device))
+
+    def check() -> None:
+        done.synchronize()
+        _raise_if_flagged(word)
+    return check
+
+
 def quantize_kv_into(cache: dict, key: str, values: torch.Tensor, start: int, *,
                      assume_finite: bool = False, status: Optional[torch.Tensor] = None) -> None:
     """Quantize bf16 values [B, L, H, D] into one storage tensor at tokens

@@ -805,3 +805,45 @@ def test_join_tokens_is_torch_cat(dev, B, La, Lb, H):
         got = ops.join_tokens(a[0], second[0], a[1], second[1], a[2], second[2])
         for x, y, z in zip(got, a, second):
             assert torch.equal(x, torch.cat([y, z], dim=1))
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("-inf")])
+def test_refused_update_leaves_cache_and_mask(dev, bad):
+    """An update whose text V holds a non-finite value raises ValueError after the
+    attention was enqueued; codes, scales and cache_mask stay as they were, and
+    the same call with finite values then writes all of them."""
+    ca, kvc = pkg_module("cache_attention"), pkg_module("fp8_kv_cache")
+    g = torch.Generator(device=dev).manual_seed(9)
+    H, hist, img, txt = 2, 70, 40, 9
+    cache = kvc.make_fp8_kv_block(1, 128, H, 128, device=dev)
+    for t in cache.values():
+        t.view(torch.uint8).fill_(1)
+    mask = torch.rand(1, 128, device=dev, generator=g) > 0.5
+
+    def stream(n):
+        return [torch.randn(1, n, H, 128, device=dev, generator=g).to(torch.bfloat16) for _ in range(3)]
+
+    (qi, ki, vi), (qt, kt, vt) = stream(img), stream(txt)
+    text_mask = torch.ones(1, txt, dtype=torch.bool, device=dev)
+    text_mask[:, 5:] = False
+    before = {n: t.view(torch.uint8).clone() for n, t in cache.items()}
+    mask_before = mask.clone()
+    vbad = vt.clone()
+    vbad[0, -1, 1, 5] = bad
+    args = (cache, hist, "flash3", text_mask, True, True, mask)
+    with torch.no_grad():
+        with pytest.raises(ValueError, match="non-finite"):
+            ca.causal_attention_with_cache_mp((qi, qt), (ki, kt), (vi, vbad), *args)
+        assert all(torch.equal(t.view(torch.uint8), before[n]) for n, t in cache.items())
+        assert torch.equal(mask, mask_before)
+        ca.causal_attention_with_cache_mp((qi, qt), (ki, kt), (vi, vt), *args)
+    want = mask_before.clone()
+    want[:, hist:hist + img] = True
+    want[:, hist + img:hist + img + txt] = text_mask
+    assert torch.equal(mask, want)
+    k = torch.cat([ki, kt], 1)
+    ref = kvc.make_fp8_kv_block(1, 128, H, 128, device=dev)
+    kvc.quantize_kv_into(ref, "k", k, hist)
+    n = slice(hist, hist + img + txt)
+    assert torch.equal(cache["k"].view(torch.uint8)[:, n], ref["k"].view(torch.uint8)[:, n])
+    assert torch.equal(cache["k"].view(torch.uint8)[:, :hist], before["k"][:, :hist])
