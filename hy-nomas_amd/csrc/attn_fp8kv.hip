@@ -561,12 +561,15 @@ HN_DEVICE void load_tail_span_k(const Params& p, int64_t b, const TailOffs<NW>& 
 
 template <int NW>
 HN_DEVICE void load_tail_span_v(const TailOffs<NW>& lo, __amdgpu_buffer_rsrc_t v, uint32_t co, TailRegs<NW>& r) {
-    static_assert(Shape<NW>::VD == 4, "two dwords per key");
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(v, lo.v[j] + co, 0, 0));
-        r.v[j][0] = x.x;
-        r.v[j][1] = x.y;
+        if constexpr (Shape<NW>::VD == 8) {
+            const uint4 x = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(v, lo.v[j] + co, 0, 0));
+            r.v[j][0] = x.x; r.v[j][1] = x.y; r.v[j][2] = x.z; r.v[j][3] = x.w;
+        } else {
+            const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(v, lo.v[j] + co, 0, 0));
+            r.v[j][0] = x.x; r.v[j][1] = x.y;
+        }
     }
 }
 
@@ -983,6 +986,23 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
     // of t - 1, before the barrier ending it; one barrier per tile.
     // Scale buffer (u + NS) % 2 last served the write of tile t + NS - 2,
     // during tile t - 2 (NS = 3) or t - 1 (NS = 2), before a barrier.
+    // The tail's tiles, from n_cache on, run a loop of their own. With the general
+    // loop's geometry, per-lane addresses, unused cache writes and tail writes
+    // after the steps (and, with two stages, loads waited for on the spot), a tail
+    // tile took up to twice a steady cache tile's time; in its own loop it takes
+    // less than one (no dequantization). 11 056 queries over 11 056 cached and
+    // 11 056 tail keys with masks, in the block: 6.09 -> 5.38 ms for the whole
+    // block with the 8-wave loop; the 4-wave launch of its last 304 rows per head
+    // 228 -> 156 us.
+    const bool tail_span = tail_end > 0 && p.us1 > 0 && ((tail_end - 1) * p.us1 + D) * 2 < ((int64_t)1 << 31);
+    // Tiles below t_full exist whole and are visible to every query.
+    const int64_t tail_vis = wg_key_limit - p.kv_len, tail_full = tail_end < tail_vis ? tail_end : tail_vis;
+    const int t_full = n_cache + (tail_full > 0 ? (int)(tail_full / BKV) : 0);
+    // Descriptors spanning the tail rows of (b, h), and tile t's byte offset.
+    auto tail_rsrc = [&](const uint16_t* base) {
+        return tile_rsrc(base + b * p.us0 + h * p.us2, ((tail_end - 1) * p.us1 + D) * 2);
+    };
+    auto tail_off = [&](int t) { return (uint32_t)((int64_t)(t - n_cache) * BKV * p.us1 * 2); };
     if constexpr (NS == 2) {
         if (t_end > t_begin) {
             f32x16 sa, sb;
@@ -1057,7 +1077,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 }
                 if (t > t_begin) g = geom(t);
             }
-            for (; t < t_end; ++t) {
+            const int t_tail = tail_span && t_end > n_cache ? (t > n_cache ? t : n_cache) : t_end;
+            for (; t < t_tail; ++t) {
                 const int u = t - t_begin;
                 const uint8_t* st = smem + (u & 1) * STAGE;
                 uint8_t* nst = smem + ((u & 1) ^ 1) * STAGE;
@@ -1096,6 +1117,43 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 __syncthreads();
                 g = gn;
                 mw = mwn;
+            }
+            if (t < t_end) {
+                const __amdgpu_buffer_rsrc_t tk = tail_rsrc(p.kcur), tv = tail_rsrc(p.vcur);
+                const TailOffs<NW> to = tail_offsets<NW>(p);
+                TailRegs<NW> tregs;  // tile t + 1 (past the end: zeros that no tile reads)
+                load_tail_span_k<NW, MASK>(p, b, to, tk, tail_off(t + 1), (int64_t)(t + 1 - n_cache) * BKV, tail_end,
+                                           tregs);
+                load_tail_span_v<NW>(to, tv, tail_off(t + 1), tregs);
+                uint32_t co = tail_off(t + 2);
+                const uint32_t dco = (uint32_t)(BKV * p.us1 * 2);
+                for (; t < t_end; ++t) {
+                    const int u = t - t_begin;
+                    const uint8_t* st = smem + (u & 1) * STAGE;
+                    uint8_t* nst = smem + ((u & 1) ^ 1) * STAGE;
+                    f16x8 pf[2];
+                    rebase(mxa, c, run, o);
+                    sb = step_a(sa, c, run.nm, run.l, pf, st + ka_off + 32 * KROW, qf);
+                    mxb = step_b_with(pf, st + va_off, 0, o, sb, [&](int i) __attribute__((always_inline)) {
+                        if (i & 1) store_tail_k_part<NW>(tregs, nst, i >> 2, (i >> 1) & 1);
+                    });
+                    store_tail_mask<NW, MASK>(tregs, nst);
+                    if (t >= t_full || mw != ALL_KEYS) mxb = mask_block(sb, 1, geom(t), mw, mxb);
+                    load_tail_span_k<NW, MASK>(p, b, to, tk, co, (int64_t)(t + 2 - n_cache) * BKV, tail_end, tregs);
+                    __syncthreads();
+                    const uint64_t mwn = tile_mask<MASK>(nst);
+                    rebase(mxb, c, run, o);
+                    sa = step_a(sb, c, run.nm, run.l, pf, nst + ka_off, qf);
+                    mxa = step_b_with(pf, st + va_off, 1, o, sa, [&](int i) __attribute__((always_inline)) {
+                        store_tail_v_part<NW>(tregs, nst, i);
+                    });
+                    if (t + 1 >= t_full || mwn != ALL_KEYS)  // (unused on the last tile)
+                        mxa = mask_block(sa, 0, geom(t + 1 < t_end ? t + 1 : t), mwn, mxa);
+                    load_tail_span_v<NW>(to, tv, co, tregs);
+                    __syncthreads();
+                    co += dco;
+                    mw = mwn;
+                }
             }
         }
     } else {
@@ -1188,13 +1246,6 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 }
                 if (t > t_begin) g = geom(t);
             }
-            // The tail's tiles, [t_tail, t_end), run a loop of their own. With the
-            // general loop's geometry, per-lane addresses, unused cache writes and
-            // tail writes after the steps, a tail tile took up to twice a steady
-            // cache tile's time; here it takes less than one (no dequantization).
-            // 11 056 queries over 11 056 cached and 11 056 tail keys with masks, in
-            // the block: 6.09 -> 5.38 ms for the whole block.
-            const bool tail_span = tail_end > 0 && p.us1 > 0 && ((tail_end - 1) * p.us1 + D) * 2 < ((int64_t)1 << 31);
             const int t_tail = tail_span && t_end > n_cache ? (t > n_cache ? t : n_cache) : t_end;
             for (; t < t_tail; ++t) {
                 const int u = t - t_begin;
@@ -1241,14 +1292,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
                 mw = mwn;
             }
             if (t < t_end) {
-                const int64_t at = b * p.us0 + h * p.us2, bytes = ((tail_end - 1) * p.us1 + D) * 2;
-                const __amdgpu_buffer_rsrc_t tk = tile_rsrc(p.kcur + at, bytes), tv = tile_rsrc(p.vcur + at, bytes);
+                const __amdgpu_buffer_rsrc_t tk = tail_rsrc(p.kcur), tv = tail_rsrc(p.vcur);
                 const TailOffs<NW> to = tail_offsets<NW>(p);
-                uint32_t co = (uint32_t)((int64_t)(t + NS - n_cache) * BKV * p.us1 * 2);
+                uint32_t co = tail_off(t + NS);
                 const uint32_t dco = (uint32_t)(BKV * p.us1 * 2);
-                // Tiles below t_full exist whole and are visible to every query.
-                const int64_t vis = wg_key_limit - p.kv_len, tail_full = tail_end < vis ? tail_end : vis;
-                const int t_full = n_cache + (tail_full > 0 ? (int)(tail_full / BKV) : 0);
                 int s0 = (t - t_begin) % NS;
                 for (; t < t_end; ++t) {
                     const int s1 = s0 == NS - 1 ? 0 : s0 + 1, sw = s0 == 0 ? NS - 1 : s0 - 1;

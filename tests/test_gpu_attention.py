@@ -219,17 +219,18 @@ def test_eight_wave_short_key_ranges(O, dev, kv_len, cur_len):
            "8-wave short range")
 
 
-# The 8-wave shape's tail loop: entered from the first tile, from a partial or a
+# The tail loops: entered from the first tile, from a partial or a
 # whole last cache tile; 1 to 6 tail tiles, whole and partial; K and V strided
-# views of a QKV tensor; key masks; a chunk boundary inside the tail (queries at
-# positions 0 .. 511, chunks of 300).
+# views of a QKV tensor; key masks; a chunk boundary at key 300 (a limit for the
+# queries below it).
 @pytest.mark.parametrize("kv_len,cur_len", [(0, 1), (0, 64), (0, 192), (0, 333), (64, 65), (100, 191), (64, 320)])
 @pytest.mark.parametrize("masked,chunk", [(False, 0), (True, 0), (False, 300), (True, 300)])
-def test_eight_wave_tail_tiles(O, dev, kv_len, cur_len, masked, chunk):
-    print(f"case attn 8-wave tail kv={kv_len} cur={cur_len} masked={masked} chunk={chunk}", flush=True)
+@pytest.mark.parametrize("H", [128, 200, 3])   # 8 waves; 4 waves (Lq 100), whole ranges and split ones
+def test_tail_tiles(O, dev, H, kv_len, cur_len, masked, chunk):
+    print(f"case attn tail H={H} kv={kv_len} cur={cur_len} masked={masked} chunk={chunk}", flush=True)
     ca = pkg_module("cache_attention")
     kvc = pkg_module("fp8_kv_cache")
-    H, D, Lq = 128, 128, 512
+    D, Lq = 128, 512 if H == 128 else 100
     if kv_len:
         cache = _cache_from_chunks(dev, 1, kv_len, H, D, 40 + kv_len)
     else:
@@ -247,10 +248,10 @@ def test_eight_wave_tail_tiles(O, dev, kv_len, cur_len, masked, chunk):
     kh, vh = _dequant(O, cache, kv_len)
     kh = np.concatenate([kh, O.bf16_bits_to_f32(bf16_bits(kc[0]))], 0)
     vh = np.concatenate([vh, O.bf16_bits_to_f32(bf16_bits(vc[0]))], 0)
-    rows = np.concatenate([np.arange(0, Lq, 37), np.arange(298, 302)])
+    rows = np.concatenate([np.arange(0, Lq, 37), np.arange(298, 302) if Lq > 300 else [Lq - 1]])
     vis = O.block_causal_visible(rows, np.arange(n), chunk) if chunk else None
     _check(O, out[0, rows].float().cpu().numpy(), O.bf16_bits_to_f32(bf16_bits(q[0, rows])), kh, vh,
-           "8-wave tail", visible=vis, key_valid=valid[0].cpu().numpy())
+           "tail", visible=vis, key_valid=valid[0].cpu().numpy())
 
 
 @pytest.mark.parametrize("Lq,kv_len,H", [(128, 86400, 24), (100, 20000, 4), (1, 5000, 2)])
