@@ -40,7 +40,6 @@ SIGNATURES = {
     "hn_gated_residual": [_P, _P, _P, _I64, _P, _I64, _I64, _I64, _P],
     "hn_residual_ln_mod_quantize_fp8": [_P, _P, _P, _I64, _P, _I64, _I64, _I64, _P, _P, _I64, _F, _F,
                                         _P, _P, _P],
-    "hn_modulation": [_P, _P, _P, _P, _I64, _I64, _I64, _P],
     "hn_join_tokens": [_I, ctypes.POINTER(_P), _PI64, ctypes.POINTER(_P), _PI64, _I64, _I64, _I64, _I64,
                        _I64, ctypes.POINTER(_P), _P],
     "hn_kv_quantize": [_I, _P, _PI64, _I64, _I64, _I64, _I64, _P, _PI64, _P, _PI64, _I64, _I64,

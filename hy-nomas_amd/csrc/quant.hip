@@ -292,83 +292,6 @@ __global__ __launch_bounds__(256) void ln_mod_quantize_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// adaLN modulation out[b] = bf16(silu(vec[b]) . w^T + bias) for one or two vectors:
-// w bf16 [N, K] is read once, MOD_ROWS rows in flight per wave. A workgroup makes
-// bf16(silu(vec)) (the reference's rounding, fp32 silu) once, beside its first
-// rows' loads; each lane adds its products in storage order, then an xor
-// butterfly; fp32 throughout, one bf16 rounding after the bias. HBM bound: 18432 x 3072 (113 MB)
-// as silu, bias copy and library GEMM 77 us -> 34 us.
-constexpr int MOD_ROWS = 4;
-
-template <int CPL, int NB>
-__global__ __launch_bounds__(256) void modulation_kernel(const uint16_t* __restrict__ vec, const uint16_t* __restrict__ w,
-                                                         const uint16_t* __restrict__ bias, uint16_t* __restrict__ out,
-                                                         int64_t N, int64_t K) {
-    const int lane = threadIdx.x & 63, nchunks = (int)(K >> 3);
-    __shared__ uint4 xs[NB][CPL * 64];
-    uint4 m[MOD_ROWS][CPL], x[NB][CPL];
-    auto load = [&](int64_t n0) {
-#pragma unroll
-        for (int r = 0; r < MOD_ROWS; ++r) {
-            const int64_t n = n0 + r < N ? n0 + r : N - 1;
-#pragma unroll
-            for (int i = 0; i < CPL; ++i) {
-                const int c = lane + i * 64;
-                m[r][i] = make_uint4(0u, 0u, 0u, 0u);
-                if (c < nchunks) m[r][i] = *reinterpret_cast<const uint4*>(w + n * K + (int64_t)c * 8);
-            }
-        }
-    };
-    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), waves = (int64_t)gridDim.x * 4;
-    load(wave * MOD_ROWS);  // in flight beside the activation, which the workgroup shares
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-        for (int c = threadIdx.x; c < CPL * 64; c += 256) {
-            uint4 o4 = make_uint4(0u, 0u, 0u, 0u);
-            if (c < nchunks) {
-                const uint4 v = *reinterpret_cast<const uint4*>(vec + b * K + (int64_t)c * 8);
-                const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
-                uint32_t o[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float lo = bf16_lo(vw[j]), hi = bf16_hi(vw[j]);
-                    o[j] = f32x2_to_bf16x2(lo / (1.0f + expf(-lo)), hi / (1.0f + expf(-hi)));
-                }
-                o4 = make_uint4(o[0], o[1], o[2], o[3]);
-            }
-            xs[b][c] = o4;
-        }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int i = 0; i < CPL; ++i) x[b][i] = xs[b][lane + i * 64];
-    for (int64_t n0 = wave * MOD_ROWS; n0 < N; n0 += waves * MOD_ROWS) {
-        if (n0 != wave * MOD_ROWS) load(n0);
-#pragma unroll
-        for (int r = 0; r < MOD_ROWS; ++r)
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                float acc = 0.0f;
-#pragma unroll
-                for (int i = 0; i < CPL; ++i) {
-                    const uint32_t a[4] = {m[r][i].x, m[r][i].y, m[r][i].z, m[r][i].w};
-                    const uint32_t v[4] = {x[b][i].x, x[b][i].y, x[b][i].z, x[b][i].w};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        acc = fmaf(bf16_lo(a[j]), bf16_lo(v[j]), acc);
-                        acc = fmaf(bf16_hi(a[j]), bf16_hi(v[j]), acc);
-                    }
-                }
-                acc = group_sum<64>(acc);
-                const int64_t n = n0 + r;
-                if (lane == 0 && n < N)
-                    out[b * N + n] = f32_to_bf16_bits(acc + (bias ? bf16_bits_to_f32(bias[n]) : 0.0f));
-            }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Up to three token concatenations out[i] = [a[i] | b[i]] along dim 1 of [B, L, H,
 // 128] bf16 tensors (a stream pair's Q, K and V before the cached attention), in
 // one launch: 16 lanes move a (token, head) row of 256 bytes, 4 rows in flight
@@ -1010,27 +933,4 @@ extern "C" int hn_join_tokens(int n, const void* const* a, const int64_t* as, co
     const dim3 grid((unsigned)stream_grid((j.rows + 63) / 64, 16 / n), (unsigned)n);
     join_tokens_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(j);
     return check_launch("hn_join_tokens");
-}
-
-extern "C" int hn_modulation(const void* vec, const void* weight, const void* bias, void* out, int64_t B, int64_t N,
-                             int64_t K, void* stream) {
-    HN_REQUIRE((B == 1 || B == 2) && N > 0 && K > 0 && K % 8 == 0 && K <= 4096, HN_E_ARG,
-               "hn_modulation: 1 or 2 vectors of K <= 4096 values, a multiple of 8");
-    HN_REQUIRE(vec && weight && out && aligned(vec, 16) && aligned(weight, 16) && aligned(bias, 2) && aligned(out, 2),
-               HN_E_ARG, "hn_modulation: null or misaligned pointer");
-    if (const int rc = require_gfx950("hn_modulation"); rc != HN_OK) return rc;
-    const int per_lane = (int)((K / 8 + 63) / 64);  // 16-byte chunks per lane, <= 8
-    const dim3 grid((unsigned)stream_grid((N + 4 * MOD_ROWS - 1) / (4 * MOD_ROWS), 8));
-#define HN_MOD_CASE(C)                                                                                            \
-    if (per_lane <= C) {                                                                                          \
-        const uint16_t *v = (const uint16_t*)vec, *w = (const uint16_t*)weight, *b = (const uint16_t*)bias;       \
-        if (B == 1) modulation_kernel<C, 1><<<grid, 256, 0, (hipStream_t)stream>>>(v, w, b, (uint16_t*)out, N, K); \
-        else modulation_kernel<C, 2><<<grid, 256, 0, (hipStream_t)stream>>>(v, w, b, (uint16_t*)out, N, K);        \
-        return check_launch("hn_modulation");                                                                     \
-    }
-    HN_MOD_CASE(2)
-    HN_MOD_CASE(6)
-    HN_MOD_CASE(8)
-#undef HN_MOD_CASE
-    return fail(HN_E_ARG, "hn_modulation: unsupported width");
 }

@@ -112,7 +112,7 @@ class FP8DiTBlock(nn.Module):
         B, L, C = x.shape
         H, D = self.heads, self.head_dim
         with stage("modulation"):
-            parts = ops.modulation(vec, mod).chunk(6, dim=-1)
+            parts = F.linear(F.silu(vec), mod.weight, mod.bias).chunk(6, dim=-1)
             if self._fused(qkv_linear):
                 qx, sx = ops.ln_modulate_quantize_fp8(x, parts[0], parts[1], 1e-6)
             else:

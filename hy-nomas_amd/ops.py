@@ -181,38 +181,6 @@ def _(x, shift, scale, eps=1e-6, amax_floor=1e-4):
     return x.new_empty((n, x.shape[2]), dtype=FP8), x.new_empty((n,), dtype=torch.float32)
 
 
-def modulation(vec, linear: torch.nn.Linear):
-    """F.linear(F.silu(vec), linear.weight, linear.bias) of bf16 [B, K] vectors: one
-    kernel for one or two of them without autograd, else the two torch ops."""
-    w, b = linear.weight, linear.bias
-    if (vec.is_cuda and vec.ndim == 2 and vec.shape[0] in (1, 2) and vec.shape[1] <= 4096 and vec.shape[1] % 8 == 0
-            and type(linear) is torch.nn.Linear and w.device == vec.device and w.is_contiguous()
-            and vec.shape[1] == w.shape[1] and vec.dtype == w.dtype == torch.bfloat16
-            and (b is None or (b.dtype == w.dtype and b.device == w.device and b.is_contiguous()))
-            and w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled("cuda")
-            and not (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (vec, w, b)))):
-        return _modulation_op(vec, w, b)
-    return torch.nn.functional.linear(torch.nn.functional.silu(vec), w, b)
-
-
-@eager_op("hy_nomas_amd::modulation")
-def _modulation_op(vec: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
-    vec = vec.contiguous()
-    if vec.data_ptr() % 16:
-        vec = vec.clone()
-    out = torch.empty((vec.shape[0], weight.shape[0]), dtype=torch.bfloat16, device=vec.device)
-    with _on(vec.device):
-        L.check(L.load().hn_modulation(vec.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(),
-                                       out.data_ptr(), vec.shape[0], weight.shape[0], weight.shape[1], _stream(vec)),
-                "hn_modulation")
-    return out
-
-
-@_modulation_op.register_fake
-def _(vec, weight, bias):
-    return vec.new_empty((vec.shape[0], weight.shape[0]))
-
-
 def _residual_args(x, y, gate, what: str):
     """Checks of x and y bf16 [B, L, C] and gate bf16 [B, C]; contiguous x, y and gate."""
     _gpu(x, y, gate)

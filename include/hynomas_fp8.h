@@ -104,13 +104,6 @@ int hn_join_tokens(int n, const void *const *a, const int64_t *as, const void *c
                    const int64_t *bs, int64_t B, int64_t La, int64_t Lb, int64_t H, int64_t D,
                    void *const *out, void *stream);
 
-/* adaLN modulation out = bf16(silu(vec) weight^T + bias), silu(vec) rounded to bf16:
- * vec bf16 [B, K] (B 1 or 2), weight bf16 [N, K], bias bf16 [N] or NULL, out bf16 [B,
- * N], all contiguous; K % 8 == 0, K <= 4096. The block's parts of
- * nomas_compile_prepost.py:29-72. */
-int hn_modulation(const void *vec, const void *weight, const void *bias, void *out, int64_t B,
-                  int64_t N, int64_t K, void *stream);
-
 /* 128x128 blockwise FP8 quantization, rows zero-padded to a multiple of 128.
  * x: bf16 [rows, cols] contiguous; q: e4m3 [rows, cols]; scale: fp32
  * [ceil(rows/128), cols/128]; cols % 128 == 0. Scale rule HN_SCALE_CLAMP with

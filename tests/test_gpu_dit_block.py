@@ -297,6 +297,26 @@ def test_ar_chunk_loop_structure(dev):
     assert torch.isfinite(x1).all()
 
 
+@pytest.mark.parametrize("batch", [1, 2])
+def test_block_modulation_is_the_references_ops(dev, batch):
+    """Both streams' six parts are the bits of F.linear(F.silu(vec), weight, bias)
+    (nomas_compile_prepost.py:29-38): a sum in another order moves single parts by a
+    bf16 step, and codes downstream with them."""
+    print(f"case dit block modulation batch={batch}", flush=True)
+    db = pkg_module("dit_block")
+    hidden, heads, L = 3072, 24, 16
+    g = torch.Generator(device=dev).manual_seed(29)
+    blk = db.FP8DiTBlock(hidden, heads, device=dev, generator=g, text=True)
+    x = torch.randn(batch, L, hidden, device=dev, generator=g).to(torch.bfloat16)
+    vec = torch.randn(batch, hidden, device=dev, generator=g).to(torch.bfloat16)
+    cos, sin = db.rope_tables(1, 4, 4, device=dev)
+    with torch.no_grad():
+        parts = blk.pre_attention(x, vec, cos, sin)[3]
+        tparts = blk.pre_attention_txt(x, vec)[3]
+        for got, mod in ((parts, blk.mod), (tparts, blk.txt_mod)):
+            assert torch.equal(torch.cat(got, -1), F.linear(F.silu(vec), mod.weight, mod.bias))
+
+
 # ---------------------------------------------------------------------------
 # The text stream of the double-stream block (nomas_compile_prepost.py:37-38,
 # 55-63, 90-98) and its cached attention over [history | img | txt]

@@ -441,27 +441,3 @@ def test_kv_write_touches_only_its_slot(dev, fmt):
         b = t.view(torch.uint8)
         assert bool((b[:, :40] == 0x5A).all()) and bool((b[:, 70:] == 0x5A).all()), name
         assert not bool((b[:, 40:70] == 0x5A).all()), name
-
-
-@pytest.mark.parametrize("B,K,N", [(1, 3072, 18432), (2, 512, 3072), (1, 8, 5), (2, 4096, 37), (1, 1032, 130)])
-@pytest.mark.parametrize("bias", [True, False])
-def test_modulation_kernel(dev, B, K, N, bias):
-    """Against silu (rounded to bf16, as F.silu gives it) and the product in 64 bits:
-    within half a bf16 step of the value plus the fp32 sum's K 2^-24 of the
-    products' magnitudes; three vectors take the torch ops."""
-    print(f"case modulation {B}x{K}x{N} bias={bias}", flush=True)
-    ops = pkg_module("ops")
-    g = torch.Generator(device=dev).manual_seed(K + N)
-    lin = torch.nn.Linear(K, N, bias=bias, device=dev, dtype=torch.bfloat16).requires_grad_(False)
-    vec = (torch.randn(B, K, device=dev, generator=g) * 3).to(torch.bfloat16)
-    x, w = torch.nn.functional.silu(vec).double(), lin.weight.double()
-    ref = x @ w.t() + (lin.bias.double() if bias else 0.0)
-    size = x.abs() @ w.abs().t() + (lin.bias.double().abs() if bias else 0.0)
-    got = ops.modulation(vec, lin)
-    assert got.dtype == torch.bfloat16 and got.shape == (B, N)
-    # silu's own fp32 rounding may land one bf16 step off F.silu's in rare places
-    bound = ref.abs() * 2.0 ** -8 + size * (K * 2.0 ** -24 + 2.0 ** -8 / K ** 0.5)
-    assert bool(((got.double() - ref).abs() <= bound).all())
-    three = vec[:1].repeat(3, 1)
-    assert torch.equal(ops.modulation(three, lin),
-                       torch.nn.functional.linear(torch.nn.functional.silu(three), lin.weight, lin.bias))
