@@ -557,18 +557,20 @@ def _(q, k, v, q_weight, k_weight, cos, sin, eps, k_codes, v_codes, k_scale, v_s
 # --------------------------------------------------------------------------
 # attention
 
-def _joinable(t: torch.Tensor) -> bool:
-    return (t.dtype == torch.bfloat16 and t.ndim == 4 and t.shape[3] == 128 and t.stride(3) == 1
-            and all(s % 8 == 0 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0)
-
-
 def join_tokens(qa, qb, ka, kb, va, vb):
     """torch.cat([a, b], dim=1) of the q, k and v of two token streams, bf16 [B, L,
-    H, 128] each, in one kernel where it reads their layout."""
+    H, 128] each, in one kernel where it reads their layout. Only metadata that a
+    trace holds (types, shapes, strides) is looked at here; addresses are looked
+    at in the op, so that a compiled caller keeps one graph."""
     pairs = (qa, qb, ka, kb, va, vb)
-    if (all(t.is_cuda and t.device == qa.device and _joinable(t) for t in pairs)
-            and all(t.shape == qa.shape for t in (ka, va)) and all(t.shape == qb.shape for t in (kb, vb))
-            and (qa.shape[0], qa.shape[2]) == (qb.shape[0], qb.shape[2])):
+    joinable = True
+    for t in pairs:
+        if not (t.is_cuda and t.device == qa.device and t.dtype == torch.bfloat16 and t.ndim == 4
+                and t.shape[3] == 128 and t.stride(3) == 1 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0
+                and t.stride(2) % 8 == 0):
+            joinable = False
+    if (joinable and ka.shape == qa.shape and va.shape == qa.shape and kb.shape == qb.shape
+            and vb.shape == qb.shape and qa.shape[0] == qb.shape[0] and qa.shape[2] == qb.shape[2]):
         return _join_tokens_op(*pairs)
     return torch.cat([qa, qb], dim=1), torch.cat([ka, kb], dim=1), torch.cat([va, vb], dim=1)
 
@@ -576,6 +578,8 @@ def join_tokens(qa, qb, ka, kb, va, vb):
 @eager_op("hy_nomas_amd::join_tokens")
 def _join_tokens_op(qa: torch.Tensor, qb: torch.Tensor, ka: torch.Tensor, kb: torch.Tensor, va: torch.Tensor,
                     vb: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    if any(t.data_ptr() % 16 for t in (qa, qb, ka, kb, va, vb)):  # the kernel loads 16 bytes
+        return torch.cat([qa, qb], dim=1), torch.cat([ka, kb], dim=1), torch.cat([va, vb], dim=1)
     B, La, H, D = qa.shape
     Lb = qb.shape[1]
     out = tuple(torch.empty((B, La + Lb, H, D), dtype=torch.bfloat16, device=qa.device) for _ in range(3))

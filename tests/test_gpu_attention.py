@@ -808,6 +808,19 @@ def test_join_tokens_is_torch_cat(dev, B, La, Lb, H):
             assert torch.equal(x, torch.cat([y, z], dim=1))
 
 
+def test_join_tokens_of_a_misaligned_source(dev):
+    """A source 2 bytes past a 16-byte boundary, in a layout the kernel reads otherwise:
+    the op concatenates it by torch."""
+    ops = pkg_module("ops")
+    g = torch.Generator(device=dev).manual_seed(3)
+    a = torch.randn(3, 1, 40, 2, 128, device=dev, generator=g).to(torch.bfloat16)
+    b = torch.randn(3 * 7 * 256 + 1, device=dev, generator=g).to(torch.bfloat16)[1:].view(3, 1, 7, 2, 128)
+    assert b.data_ptr() % 16 == 2
+    got = ops.join_tokens(a[0], b[0], a[1], b[1], a[2], b[2])
+    for i in range(3):
+        assert torch.equal(got[i], torch.cat([a[i], b[i]], dim=1))
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("-inf")])
 def test_refused_update_leaves_cache_and_mask(dev, bad):
     """An update whose text V holds a non-finite value raises ValueError after the

@@ -428,6 +428,32 @@ def test_block_text_stream(dev, update_cache):
         assert torch.isfinite(_cpu(gotv)).all() and rel <= OUTPUT_REL_L2
 
 
+def _text_block(dev, seed):
+    """A block with text over a masked history: (block, inputs, its call's keywords)."""
+    db = pkg_module("dit_block")
+    _, cache, hist, _, _, img, vec, cos, sin, L = _setup(dev)
+    g = torch.Generator(device=dev).manual_seed(seed)
+    blk = db.FP8DiTBlock(512, 4, device=dev, generator=g, text=True)
+    txt = torch.randn(1, 24, 512, device=dev, generator=g).to(torch.bfloat16)
+    text_mask = torch.arange(24, device=dev)[None] < 19
+    cache_mask = torch.rand(1, cache["k"].shape[1], device=dev, generator=g) > 0.1
+    return blk, (img, txt, vec, cos, sin, cache, hist), dict(text_mask=text_mask, cache_mask=cache_mask)
+
+
+def test_block_with_text_compiled_is_eager(dev):
+    """A denoising pass compiled as one graph gives the eager call's bits."""
+    print("case dit block compiled", flush=True)
+    blk, (img, txt, vec, cos, sin, cache, hist), masks = _text_block(dev, 41)
+
+    def call(i, t, v):
+        return blk(i, v, cos, sin, cache, hist, txt=t, vec_txt=v, **masks)
+    with torch.no_grad():
+        ref = call(img, txt, vec)
+        got = torch.compile(call, backend="aot_eager", fullgraph=True)(img, txt, vec)
+    torch._dynamo.reset()
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+
+
 def test_ar_chunk_loop_with_text(dev):
     """A 2-block model with the text stream over two chunks: every write pass
     stores img + txt K/V, the cache masks hold the padded text keys invalid,
