@@ -103,7 +103,11 @@ def read_flag_later(status: torch.Tensor):
     function that waits for the read alone and raises ValueError if the write
     was refused. Work enqueued in between keeps the GPU busy: waiting for the
     word at once drains the stream, and the host then enqueues behind an idle
-    GPU (about 170 us in a block's write pass)."""
+    GPU (about 170 us in a block's write pass). A compiled caller reads the word
+    at once: pinned memory and events do not trace (inductor refuses both)."""
+    if torch.compiler.is_compiling():
+        _raise_if_flagged(status)
+        return lambda: None
     word = torch.empty(1, dtype=torch.int32, pin_memory=True)
     word.copy_(status[:1], non_blocking=True)
     done = torch.cuda.Event()

@@ -71,3 +71,21 @@ def test_block_halves_and_seam_are_one_graph_each(traced):
         return ca.causal_attention_with_cache_mp((iq, tq), (ik, tk), (iv, tv), x["cache"], 132, "flash3",
                                                  x["masks"]["text_mask"], False, True, x["masks"]["cache_mask"])
     assert graphs(seam, *img, *txt) == 1
+
+
+def test_write_verdict_under_compile_is_read_at_once():
+    """A compiled write pass raises on its status word without pinned memory or events
+    (neither exists in this process, and inductor traces neither)."""
+    kvc = pkg_module("fp8_kv_cache")
+
+    def call(status, x):
+        refused = kvc.read_flag_later(status)
+        y = x + 1
+        refused()
+        return y
+    torch._dynamo.reset()
+    compiled = torch.compile(call, backend="eager")
+    assert torch.equal(compiled(torch.zeros(1, dtype=torch.int32), torch.ones(2)), torch.full((2,), 2.0))
+    with pytest.raises(ValueError, match="non-finite"):
+        compiled(torch.ones(1, dtype=torch.int32), torch.ones(2))
+    torch._dynamo.reset()

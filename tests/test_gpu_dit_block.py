@@ -454,6 +454,35 @@ def test_block_with_text_compiled_is_eager(dev):
     assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
 
 
+def test_compiled_update_of_the_cached_attention(dev):
+    """The seam's write pass, compiled: the eager pass's outputs,
+    cache and mask bits, and a non-finite value is refused."""
+    print("case compiled update", flush=True)
+    ca = pkg_module("cache_attention")
+    results = []
+    for compiled in (False, True):
+        blk, (img, txt, vec, cos, sin, cache, hist), masks = _text_block(dev, 43)
+        L = img.shape[1]
+        g = torch.Generator(device=dev).manual_seed(44)
+        q, k, v = (torch.randn(1, L, 4, 128, device=dev, generator=g).to(torch.bfloat16) for _ in range(3))
+        tq, tk, tv = (torch.randn(1, 24, 4, 128, device=dev, generator=g).to(torch.bfloat16) for _ in range(3))
+
+        def call(q, tq, k, tk, v, tv):
+            return ca.causal_attention_with_cache_mp((q, tq), (k, tk), (v, tv), cache, hist, "flash3",
+                                                     masks["text_mask"], True, True, masks["cache_mask"])
+        fn = torch.compile(call, backend="aot_eager") if compiled else call
+        with torch.no_grad():
+            out = fn(q, tq, k, tk, v, tv)
+            state = [t.view(torch.uint8).clone() for t in cache.values()] + [masks["cache_mask"].clone()]
+            v[0, 3, 1, 5] = float("nan")
+            with pytest.raises(ValueError, match="non-finite"):
+                fn(q, tq, k, tk, v, tv)
+        results.append([*out, *state])
+    torch._dynamo.reset()
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
 def test_ar_chunk_loop_with_text(dev):
     """A 2-block model with the text stream over two chunks: every write pass
     stores img + txt K/V, the cache masks hold the padded text keys invalid,
