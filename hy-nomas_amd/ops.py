@@ -181,14 +181,20 @@ def _(x, shift, scale, eps=1e-6, amax_floor=1e-4):
     return x.new_empty((n, x.shape[2]), dtype=FP8), x.new_empty((n,), dtype=torch.float32)
 
 
+def _rows16(t: torch.Tensor) -> torch.Tensor:
+    """t contiguous and 16-byte aligned, as the kernels load it (a copy where it is not)."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 def _residual_args(x, y, gate, what: str):
-    """Checks of x and y bf16 [B, L, C] and gate bf16 [B, C]; contiguous x, y and gate."""
+    """Checks of x and y bf16 [B, L, C] and gate bf16 [B, C]; x, y and gate for the kernel."""
     _gpu(x, y, gate)
     if x.dtype != torch.bfloat16 or y.dtype != torch.bfloat16 or gate.dtype != torch.bfloat16:
         raise TypeError(f"{what} expects bf16 tensors")
     if x.ndim != 3 or y.shape != x.shape or gate.shape != (x.shape[0], x.shape[2]):
         raise ValueError(f"{what}: x and y [B, L, C] with gate [B, C]")
-    return x.contiguous(), y.contiguous(), gate.contiguous()
+    return _rows16(x), _rows16(y), _rows16(gate)
 
 
 @eager_op("hy_nomas_amd::gated_residual", mutates_args=())

@@ -297,6 +297,33 @@ def test_ar_chunk_loop_structure(dev):
     assert torch.isfinite(x1).all()
 
 
+@pytest.mark.parametrize("which", ["x", "gates", "both"])
+def test_post_attention_of_misaligned_operands(dev, which):
+    """x and the two gates are operands of tensor ops in the reference, at any address:
+    2 bytes past a 16-byte boundary they give the aligned call's bits."""
+    print(f"case dit block post misaligned {which}", flush=True)
+    db = pkg_module("dit_block")
+    g = torch.Generator(device=dev).manual_seed(31)
+    B, L, C = 2, 37, 512
+    blk = db.FP8DiTBlock(C, 4, device=dev, generator=g)
+
+    def rand(*shape):
+        return torch.randn(*shape, device=dev, generator=g).to(torch.bfloat16)
+
+    def shifted(t):
+        u = torch.empty(t.numel() + 1, dtype=t.dtype, device=dev)[1:].view(t.shape)
+        assert u.data_ptr() % 16 == 2
+        return u.copy_(t)
+
+    x, attn, parts = rand(B, L, C), rand(B, L, 4, 128), [rand(B, C) for _ in range(6)]
+    with torch.no_grad():
+        ref = blk.post_attention(x, attn, parts)
+        gates = which != "x"
+        moved = [shifted(p) if gates and i in (2, 5) else p for i, p in enumerate(parts)]
+        got = blk.post_attention(x if which == "gates" else shifted(x), attn, moved)
+    assert torch.equal(got, ref)
+
+
 @pytest.mark.parametrize("batch", [1, 2])
 def test_block_modulation_is_the_references_ops(dev, batch):
     """Both streams' six parts are the bits of F.linear(F.silu(vec), weight, bias)
