@@ -154,6 +154,8 @@ __global__ __launch_bounds__(256) void quantize_rows_wide_kernel(
 // (bf16 tensor ops of nomas_compile_prepost.py:75-88), written to `out`. As
 // separate kernels the product, the sum and the LayerNorm read or write 8 bf16
 // rows and one row of codes; here 3 and one: 10800 x 3072 89 -> 58 us.
+// `out` may be x itself (each wave stores a row it has loaded), so x is not
+// __restrict__ in the kernels that take a Residual.
 struct Residual {
     const uint16_t* y;
     const uint16_t* gate;
@@ -176,7 +178,7 @@ HN_DEVICE uint4 gated_residual8(const uint4& x, const uint4& y, const uint4& g) 
 
 template <int CPL, bool FULL, bool RES>
 __global__ __launch_bounds__(256) void ln_mod_quantize_kernel(
-    const uint16_t* __restrict__ x, int64_t rows, int64_t cols, int64_t rows_per_batch,
+    const uint16_t* x, int64_t rows, int64_t cols, int64_t rows_per_batch,
     const uint16_t* __restrict__ shift, const uint16_t* __restrict__ scl, int64_t mod_stride, float eps,
     float amax_floor, uint8_t* __restrict__ q, float* __restrict__ scale, Residual res) {
 #pragma clang fp contract(off)
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(256) void join_tokens_kernel(JoinArgs a) {
 // in flight together. HBM bound: 3 bf16 rows, where the two tensor ops moved 5;
 // 10800 x 3072 59 -> 37 us.
 template <int CPL>
-__global__ __launch_bounds__(256) void gated_residual_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t cols,
+__global__ __launch_bounds__(256) void gated_residual_kernel(const uint16_t* x, int64_t rows, int64_t cols,
                                                              int64_t rows_per_batch, Residual res) {
     const int lane = threadIdx.x & 63;
     const int nchunks = (int)(cols >> 3);

@@ -89,7 +89,8 @@ int hn_ln_mod_quantize_fp8(const void *x, int64_t rows, int64_t cols, int64_t ro
 int hn_gated_residual(const void *x, const void *y, const void *gate, int64_t gate_stride, void *out,
                       int64_t rows, int64_t cols, int64_t rows_per_batch, void *stream);
 
-/* hn_gated_residual into x_out, then hn_ln_mod_quantize_fp8 of it, in one pass. */
+/* hn_gated_residual into x_out (which may be x), then hn_ln_mod_quantize_fp8 of it,
+ * in one pass. */
 int hn_residual_ln_mod_quantize_fp8(const void *x, const void *y, const void *gate, int64_t gate_stride,
                                     void *x_out, int64_t rows, int64_t cols, int64_t rows_per_batch,
                                     const void *shift, const void *scale_mod, int64_t mod_stride,

@@ -267,6 +267,26 @@ def test_gated_residual_kernels(dev, B, L, C):
         ops.gated_residual(x, y.float(), gate)
 
 
+def test_gated_residual_in_place(dev):
+    """Through the C API, whose `out` may be x: the residual alone and with the
+    LayerNorm, written over x, equal the out-of-place calls."""
+    ops, L = pkg_module("ops"), pkg_module("_lib")
+    lib, st = L.load(), torch.cuda.current_stream().cuda_stream
+    B, Lt, C = 2, 301, 3080
+    x, sh, sc = _ln_inputs(dev, B, Lt, C, 17)
+    y, _, gate = _ln_inputs(dev, B, Lt, C, 18)
+    out, q, s = ops.ln_modulate_quantize_fp8(x, sh, sc, 1e-6, residual=(y, gate))
+    alone, fused = x.clone(), x.clone()
+    q2, s2 = torch.empty_like(q), torch.empty_like(s)
+    L.check(lib.hn_gated_residual(alone.data_ptr(), y.data_ptr(), gate.data_ptr(), C, alone.data_ptr(), B * Lt, C, Lt,
+                                  st), "hn_gated_residual")
+    L.check(lib.hn_residual_ln_mod_quantize_fp8(
+        fused.data_ptr(), y.data_ptr(), gate.data_ptr(), C, fused.data_ptr(), B * Lt, C, Lt, sh.data_ptr(),
+        sc.data_ptr(), C, 1e-6, 1e-4, q2.data_ptr(), s2.data_ptr(), st), "hn_residual_ln_mod_quantize_fp8")
+    assert torch.equal(alone, out) and torch.equal(fused, out)
+    assert np.array_equal(u8(q2), u8(q)) and torch.equal(s2, s)
+
+
 def test_ln_modulate_quantize_matches_unfused_torch_path(dev):
     """Against F.layer_norm + the bf16 modulate ops + quantize_rows_fp8 on the GPU
     (torch's own LayerNorm summation): codes agree except where a LayerNorm output
