@@ -209,6 +209,34 @@ def test_ops_refuse_cpu_tensors():
         ops.linear_fp8(x, torch.zeros(128, 128, dtype=torch.float8_e4m3fn), torch.ones(128))
 
 
+def test_ops_infer_shapes_of_meta_tensors():
+    """Meta tensors meet each op's fake kernel (shape inference without a GPU)."""
+    torch = pytest.importorskip("torch")
+    ops, kvc, ca = pkg_module("ops"), pkg_module("fp8_kv_cache"), pkg_module("cache_attention")
+
+    def m(*shape, dtype=torch.bfloat16):
+        return torch.empty(*shape, dtype=dtype, device="meta")
+
+    f8, f32 = torch.float8_e4m3fn, torch.float32
+    w, s = m(384, 256, dtype=f8), m(384, dtype=f32)
+    assert [tuple(t.shape) for t in ops.quantize_rows_fp8(m(4, 256))] == [(4, 256), (4,)]
+    assert [tuple(t.shape) for t in ops.quantize_blockwise_fp8(m(4, 256))] == [(4, 256), (1, 2)]
+    assert ops.linear_fp8(m(4, 256), w, s).shape == (4, 384)
+    assert ops.gemm_fp8_rowcol(m(4, 256, dtype=f8), w, m(4, dtype=f32), s).shape == (4, 384)
+    assert ops.gemm_fp8_blockwise(m(4, 256, dtype=f8), w, m(1, 2, dtype=f32), m(3, 2, dtype=f32)).shape == (4, 384)
+    x, row = m(1, 4, 256), m(1, 256)
+    assert ops.ln_modulate_quantize_fp8(x, row, row)[0].shape == (4, 256)
+    out, q, _ = ops.ln_modulate_quantize_fp8(x, row, row, residual=(x, row))
+    assert out.shape == x.shape and q.shape == (4, 256)
+    assert ops.gated_residual(x, x, row).shape == x.shape
+    cache = {n: m(1, 64, 2, 128, dtype=f8) for n in ("k", "v")}
+    cache.update({n + "_scale": m(1, 64, 2, 1, dtype=f32) for n in ("k", "v")})
+    kv = m(1, 5, 2, 128)
+    kvc.quantize_kv_pair_into(cache, kv, kv, 0, status=m(1, dtype=torch.int32))
+    assert ops.kv_dequantize(cache["k"], cache["k_scale"], 10).shape == (1, 10, 2, 128)
+    assert ca.chunk_attention(kv, cache, 20).shape == kv.shape
+
+
 def test_kv_api_validates_before_writing():
     kvc = pkg_module("fp8_kv_cache")
     cache = kvc.make_fp8_kv_block(1, 8, 2, 128, device="cpu")

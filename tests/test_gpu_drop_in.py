@@ -200,6 +200,8 @@ def test_eager_calls_past_the_dispatcher_are_the_registered_ops(dev):
         assert not ops.linear_fp8(x.clone().requires_grad_(), w, s).requires_grad
     with pytest.raises(RuntimeError):
         ops.linear_fp8(x, w, s, None, 0.5)                       # act: int in the schema
+    # a view whose negation is pending: the dispatcher resolves it
+    assert torch.equal(ops.linear_fp8(torch._neg_view(x), w, s), -y)
     cache = kvc.make_fp8_kv_block(1, 64, 2, 128, device=dev)
     kv = torch.randn(1, 8, 2, 128, device=dev, generator=g).to(torch.bfloat16)
     before = {n: t._version for n, t in cache.items()}
