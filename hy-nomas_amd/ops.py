@@ -31,8 +31,13 @@ def _gpu(*tensors) -> None:
             raise RuntimeError("hy-nomas_amd FP8 kernels need GPU tensors (there is no CPU path)")
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    if _raw_stream is None:  # a torch without the short form
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 def _on(device: torch.device):
@@ -90,7 +95,10 @@ def eager_op(name: str, mutates_args=()):
             for n, v in kw.items():
                 if not direct(v, by_name.get(n, ()), grad):
                     return False
-            return not _observed()
+            try:
+                return not _observed()
+            except AttributeError:  # a torch without one of the private names it asks
+                return False
 
         @functools.wraps(fn)
         def call(*pos, **kw):

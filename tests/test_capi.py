@@ -237,6 +237,46 @@ def test_ops_infer_shapes_of_meta_tensors():
     assert ca.chunk_attention(kv, cache, 20).shape == kv.shape
 
 
+@pytest.mark.parametrize("missing", [("autograd.forward_ad", "_current_level"), ("_C", "_len_torch_dispatch_stack"),
+                                     ("autograd", "_profiler_enabled")])
+def test_direct_calls_need_the_private_names_of_torch(monkeypatch, missing):
+    """Where torch lacks a name that tells whether a call is observed, calls go through
+    the registered op; without the short form of the current stream, the public one."""
+    torch = pytest.importorskip("torch")
+    ops = pkg_module("ops")
+
+    class Plain:                            # an argument of exactly its schema's type
+        pass
+
+    ran = []
+    monkeypatch.setitem(ops._KINDS, "Tensor", (Plain,))
+    monkeypatch.setattr(torch.library, "custom_op", lambda name, fn, mutates_args: _FakeOp(ran))
+    op = ops.eager_op("test::op")(lambda x: ran.append("direct"))
+    op(Plain())
+    owner = torch
+    for part in missing[0].split("."):
+        owner = getattr(owner, part)
+    monkeypatch.delattr(owner, missing[1])
+    op(Plain())
+    assert ran == ["direct", "op"]
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: type("S", (), {"cuda_stream": 7}))
+    assert ops._stream(torch.zeros(1)) == 7
+
+
+class _FakeOp:
+    """A registered op of schema (Tensor x) that notes its calls."""
+
+    def __init__(self, ran):
+        self.ran = ran
+        arg = type("A", (), {"name": "x", "type": "Tensor", "has_default_value": lambda self: False})()
+        self._opoverload = type("O", (), {"_schema": type("S", (), {"arguments": [arg]})})
+        self.register_fake = None
+
+    def __call__(self, x):
+        self.ran.append("op")
+
+
 def test_kv_api_validates_before_writing():
     kvc = pkg_module("fp8_kv_cache")
     cache = kvc.make_fp8_kv_block(1, 8, 2, 128, device="cpu")
