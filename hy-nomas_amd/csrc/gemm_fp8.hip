@@ -24,22 +24,18 @@
 // The MFMA's first operand is the weight tile and its second the activation
 // tile, i.e. the wave computes out^T: each lane then holds four consecutive
 // output columns n..n+3 of one row m and stores them as one 8-byte write.
-#include <algorithm>
-#include <cmath>
 #include <cstdlib>
-#include <iterator>
 #include <type_traits>
 
 #include "hn_capi_internal.h"
 #include "hn_common.h"
 #include "gemm_dma.h"
+#include "gemm_plan.h"
 
 namespace hn {
 namespace gemm {
 
-constexpr int BM = 256, BN = 256, BK = 128;
 constexpr int NT = 256;
-enum Mode { ROWCOL = 0, BLOCKWISE = 1 };
 constexpr int kMaxKT = 256;  // K <= 32768
 
 struct Params {
@@ -429,7 +425,7 @@ constexpr int O_SMEM = O_PARAM_BASE + 4 * O_PARAMS;
 constexpr int O_WC = 128;                           // columns per wave
 constexpr int O_JO = 2;                             // row blocks carried into the next tile
 constexpr int O_PASSES = 2 * O_JO;                  // overlapped passes (steps 0 .. O_PASSES - 1)
-constexpr int O_MIN_KT = O_PASSES + 3;              // + the tail step + the last two steps
+static_assert(O_MIN_KT == O_PASSES + 3, "a tile's K steps: the passes, the tail step and the last two");
 static_assert(O_SMEM <= 160 * 1024, "LDS");
 
 // Output window of one wave's 128 x wc sub-tile (first row m0w, first column
@@ -679,15 +675,6 @@ __device__ unsigned long long g_stamps[STAMP_WGS][STAMP_TILES][STAMP_PHASES];
 // shared; two stages, with one barrier after a step's loads land and one after
 // every wave has read its fragments, before that stage is refilled. The
 // epilogue is the persistent kernel's, 8 bytes (4 columns) per store.
-constexpr int TAIL_WIDE_COLS = 384;
-// Where the fused stripe gains (same-box A/B against the separate launch, two
-// runs): the north star (32 light workgroups, K 3072) 0.978x and 0.981x, QKV
-// (24, N 9216) 0.989x and 0.986x. Where it does not: past K 4096 an item
-// outlasts the light workgroups' idle round (fc2, K 12 288: 1.013x), and with
-// 8 light workgroups (out-projection, N 3072) it measured 0.991x and 1.017x.
-constexpr int64_t TAIL_WIDE_MAX_K = 4096;
-constexpr int TAIL_WIDE_MIN_LIGHT = 16;
-
 template <int JB>
 constexpr int tail_wide_stage_bytes() { return (32 * JB + TAIL_WIDE_COLS) * BK; }
 
@@ -1128,8 +1115,6 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
 // f_k = sa[mb][k] sb[nb][k] (skipped when f_k = 0), and the epilogue is
 // bf16(acc). The factors are read through the constant address space (scalar
 // loads, outside the vector-memory counter the DMA waits count).
-constexpr int TAIL_ROWS = 64;
-constexpr int TAIL_COLS = 32;
 constexpr int TAIL_STAGES = 3;
 static_assert(O_MIN_KT >= 4, "every tail wave needs a K step (K / 128 >= O_MIN_KT, at most 4 waves)");
 
@@ -1644,58 +1629,6 @@ static void launch_small_as(gemm::Params p, hipStream_t st) {
         gemm::gemm_small_kernel<MODE, HN_ACT_NONE, WR, WC, RB, CB><<<grid, block, LDS, st>>>(p, 0);
 }
 
-// The tile of a launch, by an estimate of each shape's time in us:
-//     3 + rounds * (g + K steps * c),
-// with rounds the number of tiles per CU, rounded up (64 x 64 tiles run two to
-// a CU: 0.3 more instead), and g (a tile's prologue and epilogue) and c (a
-// K step) between their values for a few tiles and for a tile on every CU,
-// where the loads from the L2s (11-15 TB/s in all) and the output's writes
-// bound them. Fitted to back-to-back calls at K 512 to 12288 and 32 to 4608
-// tiles; within 15 % of them, except where the weight comes from HBM.
-struct TileCost {
-    int tm, tn;
-    float g_low, c_low, g_full, c_full;
-};
-
-static double tile_time(const TileCost& t, int64_t M, int64_t N, int64_t K, int cus) {
-    const double tiles = (double)((M + t.tm - 1) / t.tm) * (double)((N + t.tn - 1) / t.tn);
-    const double fill = std::min(1.0, tiles / cus);
-    const double rounds = t.tm * t.tn <= 64 * 64 && tiles > cus ? tiles / cus + 0.3 : std::ceil(tiles / cus);
-    const double g = t.g_low + (t.g_full - t.g_low) * fill, c = t.c_low + (t.c_full - t.c_low) * fill;
-    return 3.0 + rounds * (g + (double)(K / gemm::BK) * c);
-}
-
-// gemm_small_kernel's shapes, per mode.
-constexpr TileCost kSmallRowcol[] = {
-    {64, 64, 1.3f, 0.18f, 1.3f, 0.18f},   {64, 128, 1.2f, 0.27f, 2.0f, 0.38f},
-    {128, 128, 2.5f, 0.34f, 2.5f, 0.60f}, {128, 192, 2.5f, 0.43f, 3.0f, 0.75f},
-    {128, 256, 2.0f, 0.57f, 4.5f, 0.86f}, {256, 192, 0.5f, 0.90f, 7.2f, 1.08f}};
-constexpr TileCost kSmallBlockwise[] = {
-    {64, 64, 1.0f, 0.25f, 1.0f, 0.25f}, {128, 128, 1.0f, 0.48f, 1.0f, 0.62f}, {128, 256, 1.4f, 0.75f, 2.0f, 1.02f}};
-// The 256 x 256 tiles of gemm_rowcol_oe_kernel (its prologues and epilogues
-// run beside other tiles' K steps, all but kBigOnce of them) and gemm_bw8_kernel.
-constexpr TileCost kBigRowcol = {256, 256, 0.0f, 1.12f, 0.0f, 1.52f};
-constexpr TileCost kBigBlockwise = {256, 256, 1.0f, 1.20f, 0.0f, 1.72f};
-constexpr double kBigOnce = 4.0;
-
-// The index of the small tile that a launch takes, or -1 for the 256 x 256
-// tiles. Below O_MIN_KT steps the persistent kernel cannot run. A last stripe
-// of at most TAIL_ROWS rows costs the 256 x 256 tiles no round. Within 3 % of
-// each other the 256 x 256 tiles win.
-static int small_plan(int mode, int64_t M, int64_t N, int64_t K, int cus) {
-    const bool row = mode == gemm::ROWCOL;
-    if (M <= gemm::TAIL_ROWS && K / gemm::BK >= (row ? gemm::O_MIN_KT : 4)) return -1;  // the tail kernel alone
-    const TileCost* const t = row ? kSmallRowcol : kSmallBlockwise;
-    const int count = row ? (int)std::size(kSmallRowcol) : (int)std::size(kSmallBlockwise);
-    int best = 0;
-    for (int i = 1; i < count; ++i)
-        if (tile_time(t[i], M, N, K, cus) < tile_time(t[best], M, N, K, cus)) best = i;
-    if (row && K / gemm::BK < gemm::O_MIN_KT) return best;
-    const int64_t tail = M % gemm::BM, Mb = tail <= gemm::TAIL_ROWS && M > tail ? M - tail : M;
-    const double big = kBigOnce + tile_time(row ? kBigRowcol : kBigBlockwise, Mb, N, K, cus);
-    return tile_time(t[best], M, N, K, cus) < 0.97 * big ? best : -1;
-}
-
 static int launch_small(const gemm::Params& p, int mode, int i, void* stream, const char* who) {
     const hipStream_t st = (hipStream_t)stream;
     if (mode == gemm::BLOCKWISE) {
@@ -1740,44 +1673,31 @@ static int gemm_launch(int mode, const void* a, const void* b, const float* sa, 
     p.M = M; p.N = N; p.K = K; p.ldc = ldc; p.act = act;
     HN_REQUIRE((M + 63) / 64 * (N / 64) <= 0x7ffffff0LL, HN_E_ARG,
                "FP8 GEMM: too many tiles");
-    if (const int i = small_plan(mode, M, N, K, device_cus()); i >= 0) return launch_small(p, mode, i, stream, who);
-    const bool persistent = mode == gemm::ROWCOL;  // K has at least O_MIN_KT steps here
-    // A last row stripe of at most TAIL_ROWS rows goes to gemm_tail_kernel (or,
-    // in persistent launches, possibly to the light workgroups), and the tiles
-    // cover only the rows above it: always in persistent launches; in
-    // blockwise ones (one tile per workgroup, one workgroup per CU) when that
-    // saves a whole round of tiles (the decoder's gate and up projections,
-    // 10 800 x 4096 -> 12 288: 2064 tiles, 9 rounds, against 2016, 8) and K
-    // has at least 4 scale blocks (a K step for each of up to 4 waves).
-    const int64_t m_tail = M % gemm::BM;
-    bool stripe = false;
-    if (m_tail > 0 && m_tail <= gemm::TAIL_ROWS) {
-        if (persistent) {
-            stripe = true;
-        } else if (mode == gemm::BLOCKWISE && K / gemm::BK >= 4) {
-            const int64_t cus = device_cus(), tn = (N + gemm::BN - 1) / gemm::BN;
-            const int64_t all = (M + gemm::BM - 1) / gemm::BM * tn, whole = M / gemm::BM * tn;
-            stripe = (all + cus - 1) / cus > (whole + cus - 1) / cus;
-        }
-    }
-    const int64_t Mt = stripe ? M - m_tail : M;
-    const int64_t tm = (Mt + gemm::BM - 1) / gemm::BM;
-    const gemm::TileCounts t = gemm::tile_counts(Mt, N, gemm::BN);
+    int wg_cap = 0;
+#ifdef HN_GEMM_PHASE_STAMPS
+    // Measurement build: HN_GEMM_WG_PER_XCD caps the workgroups per XCD (the
+    // tile queues adapt; fewer CUs busy, same tiles).
+    if (const char* e = getenv("HN_GEMM_WG_PER_XCD")) wg_cap = atoi(e);
+#endif
+    const gemm::Route r = gemm::gemm_route(mode, M, N, K, device_cus(), wg_cap);
+    if (r.small >= 0) return launch_small(p, mode, r.small, stream, who);
+    const bool stripe = r.Mt < M;
+    const int64_t Mt = r.Mt;
+    const gemm::TileCounts& t = r.tiles;
     p.tiles_m = t.tiles_m; p.tiles_n = t.tiles_n;
     p.tm_full = t.tm_full; p.tn_full = t.tn_full; p.m_tail = t.m_tail;
     p.tiles_full = t.tiles_full; p.tiles_part = t.tiles_part;
-    p.per_xcd = mode == gemm::ROWCOL ? t.per_xcd : (int)((tm * t.tiles_n + 7) / 8);
+    p.per_xcd = mode == gemm::ROWCOL ? t.per_xcd : (int)(((int64_t)t.tiles_m * t.tiles_n + 7) / 8);
     const dim3 grid((unsigned)(8 * (int64_t)p.per_xcd));
     // The tail stripe on a launch of its own, with the full M for its row
-    // clamp and stores. K is split over 2 waves, or 4 when the stripe has
-    // fewer 32-column groups than CUs.
+    // clamp and stores.
     auto launch_tail = [&]() {
         gemm::Params pt = p;
         pt.M = M;
         pt.tail_M = 0;
         const dim3 tgrid((unsigned)(N / gemm::TAIL_COLS));
         const hipStream_t st = (hipStream_t)stream;
-        const bool two = m_tail > 32, four = N / gemm::TAIL_COLS < device_cus(), gelu = act == HN_ACT_GELU_TANH;
+        const bool two = r.tail_blocks == 2, four = r.tail_waves == 4, gelu = act == HN_ACT_GELU_TANH;
         const dim3 tblock(four ? 256 : 128);
 #define HN_TAIL(A, SK, JB) gemm::gemm_tail_kernel<gemm::ROWCOL, A, SK, JB><<<tgrid, tblock, 0, st>>>(pt, Mt)
 #define HN_TAIL_BW(SK, JB) gemm::gemm_tail_kernel<gemm::BLOCKWISE, HN_ACT_NONE, SK, JB><<<tgrid, tblock, 0, st>>>(pt, Mt)
@@ -1798,38 +1718,14 @@ static int gemm_launch(int mode, const void* a, const void* b, const float* sa, 
     if (stripe && Mt == 0) return launch_tail();
     p.M = Mt;
     p.tail_M = Mt;
-    if (persistent) {
-        // Persistent: per XCD, min(queue length, CUs of the XCD) workgroups.
-        const int cus = device_cus();
-        const int per_xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
-        int wg_cap = per_xcd_cus;
-#ifdef HN_GEMM_PHASE_STAMPS
-        // Measurement build: HN_GEMM_WG_PER_XCD caps the workgroups per XCD
-        // (the tile queues adapt; fewer CUs busy, same tiles).
-        if (const char* e = getenv("HN_GEMM_WG_PER_XCD")) {
-            const int v = atoi(e);
-            if (v >= 1 && v < wg_cap) wg_cap = v;
-        }
-#endif
-        const int S = p.per_xcd < wg_cap ? p.per_xcd : wg_cap;
-        const dim3 pgrid((unsigned)(8 * S));
+    if (mode == gemm::ROWCOL) {
+        const dim3 pgrid((unsigned)(8 * r.S));
         const hipStream_t st = (hipStream_t)stream;
-        if (Mt < M) {
-            // The tail stripe rides on the light workgroups (tail_wide) when
-            // every XCD has some, at least TAIL_WIDE_MIN_LIGHT in all, there
-            // are no edge tiles, each light workgroup's share of the columns
-            // fits one item and K is at most TAIL_WIDE_MAX_K; else it has a
-            // launch of its own.
-            bool every = false;
-            const int nl = gemm::light_count(p, S, &every);
-            const int64_t cols = nl > 0 ? (N / 32 + nl - 1) / nl * 32 : 0;
-            if (p.tiles_part == 0 && every && nl >= gemm::TAIL_WIDE_MIN_LIGHT && cols <= gemm::TAIL_WIDE_COLS &&
-                K <= gemm::TAIL_WIDE_MAX_K) {
-                p.tail_M = M;
-                p.tail_cols = (int)cols;
-            } else if (const int rc = launch_tail(); rc != HN_OK) {
-                return rc;
-            }
+        if (r.tail_cols > 0) {
+            p.tail_M = M;
+            p.tail_cols = r.tail_cols;
+        } else if (stripe) {
+            if (const int rc = launch_tail(); rc != HN_OK) return rc;
         }
         if (act == HN_ACT_GELU_TANH) gemm::gemm_rowcol_oe_kernel<HN_ACT_GELU_TANH><<<pgrid, gemm::NT, 0, st>>>(p);
         else gemm::gemm_rowcol_oe_kernel<HN_ACT_NONE><<<pgrid, gemm::NT, 0, st>>>(p);

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+import gemm_shapes as S
 from conftest import assert_close_bf16, bf16_bits, pkg_module, u8
 
 pytestmark = pytest.mark.gpu
@@ -82,20 +83,15 @@ def test_linear_fp8_no_bias_and_strided_out(O, dev):
     assert (out[:, 128:] == 3.0).all()
 
 
-@pytest.mark.parametrize("M,K,N,act", [
-    (100, 1024, 256, 1),    # 256 x 192 tiles; the wave of rows 0-127 has 100 rows (four row blocks)
-    (1000, 1280, 640, 0),   # 256 x 192 tiles; the last tile's second row wave has 104 rows
-    (4964, 1024, 4224, 1),  # 256-wide tiles (340); last row tile 100 deep
-    (5092, 1024, 4224, 0),  # 256-wide tiles; last row tile 228 deep, its second row wave 100
-])
+@pytest.mark.parametrize("M,K,N,act", S.GUARD)
 def test_gemm_writes_nothing_past_m_or_n(dev, M, K, N, act):
-    """The persistent GEMM into a buffer with 64 guard rows below M and 8
-    guard columns right of N (row stride N + 8): the M x N block equals the
-    plain call's output and the guards keep their fill. Shapes whose last
-    row tile leaves a wave 97-127 rows: such a wave has four row blocks but
-    is not wholly inside, and its tile-end stores must keep their bounds
-    test (stores past row M faulted the GPU at M = 100 in a build that
-    counted blocks)."""
+    """Every small tile and the persistent kernel into a buffer with 64 guard
+    rows below M and 8 guard columns right of N (row stride N + 8): the M x N
+    block equals the plain call's output and the guards keep their fill. The
+    persistent shapes' last row tiles leave a wave 97-127 rows: such a wave has
+    four row blocks but is not wholly inside, and its tile-end stores must keep
+    their bounds test (stores past row M faulted the GPU at M = 100 in a build
+    that counted blocks)."""
     ops, L = pkg_module("ops"), pkg_module("_lib")
     print(f"case gemm guard band {M}x{K}x{N} act={act}", flush=True)
     g = torch.Generator(device=dev).manual_seed(M + N)
@@ -114,11 +110,10 @@ def test_gemm_writes_nothing_past_m_or_n(dev, M, K, N, act):
     assert bool((buf[M:] == 7.0).all()) and bool((buf[:, N:] == 7.0).all())
 
 
-@pytest.mark.parametrize("M,N,K", [(300, 256, 512), (129, 384, 1024), (4097, 128, 4096)])
+@pytest.mark.parametrize("M,N,K", S.GUARD_BLOCKWISE)
 def test_blockwise_gemm_writes_nothing_past_m(dev, M, N, K):
-    """The blockwise GEMM into a buffer 16 rows longer than its output: the
-    output rows equal the op's own result and the guard rows keep their fill
-    (last row tiles 44, 1 and 1 deep)."""
+    """Every blockwise kernel into a buffer 16 rows longer than its output: the
+    output rows equal the op's own result and the guard rows keep their fill."""
     print(f"case blockwise guard band {M}x{N}x{K}", flush=True)
     ops, L = pkg_module("ops"), pkg_module("_lib")
     pf = pkg_module("pixelumm_fp8")
@@ -133,49 +128,19 @@ def test_blockwise_gemm_writes_nothing_past_m(dev, M, N, K):
     assert torch.equal(buf[:M], ref) and bool((buf[M:] == 9.0).all())
 
 
-# K >= 7 x 128 takes the persistent kernel that carries half of each tile's
-# epilogue into the next tile's K loop. Cases: the smallest such K and the
-# largest K below it; ragged M and N (edge tiles); more tiles than CUs, so a
-# workgroup walks whole and edge tiles in turn; with and without bias / GELU.
-# A launch with fewer 256-wide tiles than CUs runs 256 x 192 tiles when that
-# gives more tiles and still one round (96 columns per wave): config 1 and
-# (64, 12288, 3072) above, and the 1000 x 640 and 700 x 1280 cases here, whose
-# last column stripes are 64 wide (one wave with two blocks, one with none) and
-# 128 wide (three blocks and one).
-@pytest.mark.parametrize("M,K,N,gelu,bias", [
-    (300, 896, 384, True, True),      # smallest K on the carried-epilogue path
-    (300, 768, 384, True, True),      # largest K below it
-    (1000, 1280, 640, True, True),    # M and N edges, 256 x 192 tiles (16)
-    (700, 1024, 1280, True, False),   # 256 x 192 tiles (21), both edges, no bias
-    (4700, 1024, 4224, True, False),  # 323 tiles: two per workgroup, both edges, no bias
-    (4700, 1024, 4224, False, True),
-    # Last row tile 132 deep: waves of rows 0-127 multiply a whole block while
-    # the stage rows they load (128-191) lie partly past M; the loads must
-    # stay inside A. On 256 x 192 tiles, and on 256-wide ones (340 tiles).
-    (132, 12288, 3072, True, True),
-    (4996, 1024, 4224, False, True),
-])
+# The persistent kernel carries half of each tile's epilogue into the next
+# tile's K loop.
+@pytest.mark.parametrize("M,K,N,gelu,bias", S.PERSISTENT)
 def test_linear_fp8_persistent_tiles(O, dev, M, K, N, gelu, bias):
     print(f"case linear persistent {M}x{K}x{N} gelu={gelu} bias={bias}", flush=True)
     rows = None if M <= 1000 else np.concatenate([np.arange(0, 64), np.arange(2300, 2364), np.arange(M - 300, M)])
     _check_linear(O, dev, M, K, N, gelu, bias=bias, rows=rows)
 
 
-# A last row stripe of at most 64 rows (M % 256) goes to gemm_tail_kernel
-# (K split over 4 waves when the stripe has fewer 32-column groups than CUs,
-# else over 2; one or two 32-row blocks) while the persistent kernel tiles the
-# rows above it; M <= 64 runs the tail kernel alone. Tails of 1, 20, 32, 33,
-# 48 and 64 rows, with and without GELU and bias.
-@pytest.mark.parametrize("M,K,N,gelu,bias", [
-    (257, 1024, 384, True, True),      # 1 tail row: one block, 4 waves
-    (288, 896, 640, False, True),      # 32 tail rows: one block
-    (289, 3072, 512, True, False),     # 33 tail rows: two blocks, no bias
-    (48, 3072, 1280, True, True),      # tail only (no persistent launch)
-    (10800, 12288, 384, False, True),  # 48 tail rows, K 12288
-    (1, 4224, 256, True, True),        # one row, K past 4096
-    (276, 4224, 8192, False, True),    # 20 tail rows, 256 column groups: K split over 2 waves
-    (576, 4352, 8192, True, True),     # 64 tail rows (two blocks), 2 waves, GELU
-])
+# A last row stripe of at most 64 rows (M % 256) beside 256 x 256 tiles goes to
+# gemm_tail_kernel while the persistent kernel tiles the rows above it; M <= 64
+# runs the tail kernel alone. Tails of 1 to 64 rows, with and without GELU and bias.
+@pytest.mark.parametrize("M,K,N,gelu,bias", S.TAIL)
 def test_linear_fp8_tail_rows(O, dev, M, K, N, gelu, bias):
     print(f"case linear tail {M}x{K}x{N} gelu={gelu} bias={bias}", flush=True)
     rows = None if M <= 1000 else np.concatenate([np.arange(0, 64), np.arange(M - 320, M)])
@@ -187,20 +152,17 @@ def test_linear_fp8_tail_rows(O, dev, M, K, N, gelu, bias):
 # stripe themselves after their last tile (tail_wide: up to 384 columns each,
 # the four waves sharing the stripe's A rows), instead of a second launch:
 # the north-star shapes (M 10800) and these.
-@pytest.mark.parametrize("M,K,N,gelu,bias", [
-    (10785, 896, 4096, True, True),    # 33 tail rows (two blocks), 96 light workgroups of 64 columns
-    (10770, 1024, 2048, False, False),  # 18 tail rows (one block)
-])
+@pytest.mark.parametrize("M,K,N,gelu,bias", S.LIGHT)
 def test_linear_fp8_tail_on_light_workgroups(O, dev, M, K, N, gelu, bias):
     print(f"case linear fused tail {M}x{K}x{N} gelu={gelu} bias={bias}", flush=True)
     rows = np.concatenate([np.arange(0, 64), np.arange(5000, 5064), np.arange(M - 320, M)])
     _check_linear(O, dev, M, K, N, gelu, bias=bias, rows=rows)
 
 
-@pytest.mark.parametrize("M,K,N,act", [(300, 1024, 384, 1), (289, 4352, 256, 0), (33, 896, 128, 1),
-                                       (10785, 896, 4096, 1), (276, 4224, 8192, 0)])
+@pytest.mark.parametrize("M,K,N,act", S.GUARD_TAIL)
 def test_gemm_tail_writes_nothing_past_m_or_n(dev, M, K, N, act):
-    """Tail stripes (44, 33 and 33 rows; the last two on 8 and 4 waves) into a
+    """Tail stripes on every form of the tail kernel, alone and beside tiles, and
+    on light workgroups (and shapes whose last rows small tiles take) into a
     buffer with 64 guard rows and 8 guard columns (row stride N + 8): the
     M x N block equals the plain call's output, the guards keep their fill,
     and a second call gives the same bits (the wave-ordered split-K sum)."""
@@ -225,9 +187,8 @@ def test_gemm_tail_writes_nothing_past_m_or_n(dev, M, K, N, act):
 
 @pytest.mark.parametrize("N", [384, 640])
 def test_gemm_rowcol_persistent_strided_out(dev, N):
-    """ldc > N on the carried-epilogue path (K = 1024): columns past N untouched.
-    N = 384 runs 256-wide tiles; N = 640 runs 256 x 192 tiles with a 64-wide
-    last stripe, whose 96-column waves must not write past their own columns."""
+    """ldc > N, no bias (64 x 64 tiles; the persistent kernel's strided outputs
+    are test_gemm_writes_nothing_past_m_or_n's): columns past N untouched."""
     ops = pkg_module("ops")
     L = pkg_module("_lib")
     ldc = N + 8
@@ -283,7 +244,7 @@ def _blockwise_check(got, expected):
     assert np.all(np.abs(got - expected) <= np.abs(expected) * 2 ** -8 + 1e-3 * np.abs(expected).max())
 
 
-@pytest.mark.parametrize("m,n,k", [(1536, 4096, 12288), (1536, 12288, 4096), (10800, 4096, 4096)])
+@pytest.mark.parametrize("m,n,k", S.DECODER)
 def test_blockwise_gemm_decoder_shapes(O, dev, m, n, k):
     """The decoder's projection shapes (pixelumm_decoder/model.py:43-53: q/o/gate/up
     and down, K 4096 and 12288), with activation K blocks whose magnitudes differ
@@ -312,7 +273,7 @@ def test_blockwise_gemm_decoder_shapes(O, dev, m, n, k):
 # over 16 column tiles (257 -> 256 tiles), and M <= 64 (the stripe alone).
 # Activation K blocks of gains up to 2^+-8, an all-zero K block and zero
 # factors (a weight K block given scale 0, and the stripe's own row block).
-@pytest.mark.parametrize("m,n,k", [(10800, 12288, 4096), (4116, 4096, 512), (48, 512, 1024), (33, 256, 4096)])
+@pytest.mark.parametrize("m,n,k", S.TAIL_BLOCKWISE)
 def test_blockwise_gemm_tail_stripe(O, dev, m, n, k):
     print(f"case blockwise tail stripe {m}x{n}x{k}", flush=True)
     pf = pkg_module("pixelumm_fp8")
@@ -339,13 +300,16 @@ def test_blockwise_gemm_tail_stripe(O, dev, m, n, k):
     assert torch.equal(pf.load_extension().gemm(qa, qb, sa, sb), got)
 
 
-def test_blockwise_gemm_zero_block_factors(O, dev):
+@pytest.mark.parametrize("m,n,k", S.ZERO_FACTORS)
+def test_blockwise_gemm_zero_block_factors(O, dev, m, n, k):
     """Block factors of 0 (an activation K block and a weight K block given scale 0
-    by the caller) contribute nothing; the other blocks are promoted as usual."""
+    by the caller, the first and the last K block among them) contribute nothing;
+    the other blocks are promoted as usual."""
+    print(f"case blockwise zero factors {m}x{n}x{k}", flush=True)
     pf = pkg_module("pixelumm_fp8")
     g = torch.Generator().manual_seed(12)
-    a = torch.randn(300, 1024, generator=g).to(torch.bfloat16)
-    b = torch.randn(384, 1024, generator=g).to(torch.bfloat16)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    b = torch.randn(n, k, generator=g).to(torch.bfloat16)
     qa, sa = pf._quantize_blockwise(a.to(dev))
     qb, sb = pf._quantize_blockwise(b.to(dev))
     sa[:, 1] = 0.0
@@ -357,16 +321,18 @@ def test_blockwise_gemm_zero_block_factors(O, dev):
     _blockwise_check(got, expected)
 
 
+@pytest.mark.parametrize("m,n,k", S.FACTOR_JUMP)
 @pytest.mark.parametrize("direction", ["up", "down"])
-def test_blockwise_gemm_factor_jump_of_2_to_60(O, dev, direction):
+def test_blockwise_gemm_factor_jump_of_2_to_60(O, dev, direction, m, n, k):
     """Adjacent K blocks whose weight factors differ by 2^60, the widest span
     the FP8Linear loader accepts: the carried accumulator's rescale by
-    f_prev / f (2^60 or 2^-60 here) stays finite, and the result matches the
-    float64 dequantize-then-matmul reference."""
+    f_prev / f (2^60 or 2^-60 here; 64 x 64 tiles have none) stays finite, and
+    the result matches the float64 dequantize-then-matmul reference."""
+    print(f"case blockwise factor jump {direction} {m}x{n}x{k}", flush=True)
     pf = pkg_module("pixelumm_fp8")
     g = torch.Generator().manual_seed(31)
-    a = torch.randn(256, 512, generator=g).to(torch.bfloat16)
-    b = torch.randn(256, 512, generator=g).to(torch.bfloat16)
+    a = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    b = torch.randn(n, k, generator=g).to(torch.bfloat16)
     qa, sa = pf._quantize_blockwise(a.to(dev))
     qb, sb = pf._quantize_blockwise(b.to(dev))
     # K blocks 2, 3 at exactly 2^60 (2^-60) times the row's smallest (largest)
@@ -377,10 +343,10 @@ def test_blockwise_gemm_factor_jump_of_2_to_60(O, dev, direction):
         sb[:, 2:] = sb[:, :2].amax(dim=1, keepdim=True) * 2.0 ** -60
     span = sb.amax(dim=1) / sb.amin(dim=1)
     assert bool((span == 2.0 ** 60).all()), span
-    pf.validate_serialized_tensors(qb, sb, (256, 512))  # within the loader's bound
+    pf.validate_serialized_tensors(qb, sb, (n, k))  # within the loader's bound
     with pytest.raises(ValueError, match="span more than 2"):
         pf.validate_serialized_tensors(qb, sb * torch.tensor([1.0, 1.0, 2.0, 2.0], device=dev) ** (
-            1 if direction == "up" else -1), (256, 512))
+            1 if direction == "up" else -1), (n, k))
     got = pf.load_extension().gemm(qa, qb, sa, sb)
     assert torch.isfinite(got.float()).all()
     expected = O.blockwise_gemm_reference(u8(qa), sa.cpu().numpy(), u8(qb), sb.cpu().numpy())
@@ -432,17 +398,7 @@ def test_fp8_linear_modules(O, dev):
         d(x.float())
 
 
-# Launches that take each shape of the small-tile kernel on 256 CUs, ragged in M
-# and (192- and 256-wide tiles) in N; K of 5 to 9 steps covers the pipeline's
-# fill and drain, and K below 896 the GELU of the unrounded value.
-@pytest.mark.parametrize("M,K,N", [
-    (100, 1024, 256), (65, 128, 384),       # 64 x 64
-    (450, 1024, 3200), (1000, 768, 2048),   # 64 x 128
-    (1000, 1024, 3072),                     # 128 x 128
-    (1025, 896, 4224),                      # 128 x 192
-    (2049, 896, 2944), (4097, 640, 3200),   # 128 x 256
-    (3000, 896, 3072), (2500, 640, 4224),   # 256 x 192
-])
+@pytest.mark.parametrize("M,K,N", S.SMALL_ROWCOL)
 @pytest.mark.parametrize("gelu", [False, True])
 def test_linear_fp8_small_tiles(O, dev, M, K, N, gelu):
     print(f"case small tiles {M}x{K}x{N} gelu={gelu}", flush=True)
@@ -450,7 +406,7 @@ def test_linear_fp8_small_tiles(O, dev, M, K, N, gelu):
     _check_linear(O, dev, M, K, N, gelu, bias=not gelu, rows=rows)
 
 
-@pytest.mark.parametrize("m,n,k", [(129, 256, 384), (1000, 1024, 2048), (2200, 640, 1920)])
+@pytest.mark.parametrize("m,n,k", S.SMALL_BLOCKWISE)
 def test_blockwise_gemm_small_tiles(O, dev, m, n, k):
     """The blockwise small tiles (64 x 64, 128 x 128, 128 x 256) with K blocks of
     gains up to 2^+-8, an all-zero activation block and zero factors."""
