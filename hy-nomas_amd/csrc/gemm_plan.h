@@ -35,17 +35,20 @@ constexpr int TAIL_WIDE_MIN_LIGHT = 16;
 // K step) between their values for a few tiles and for a tile on every CU,
 // where the loads from the L2s (11-15 TB/s in all) and the output's writes
 // bound them. Fitted to back-to-back calls at K 512 to 12288 and 32 to 4608
-// tiles; within 15 % of them, except where the weight comes from HBM.
+// tiles; within 15 % of them, except where the weight comes from HBM. Below that
+// range (K 128 to 384) the row/column pick is the fastest of the six in 19 of 21
+// shapes of 65 to 4000 rows and 384 to 3072 columns, and 14 and 17 % off it in the
+// two that give 256 x 192 tiles to every CU.
 struct TileCost {
     int tm, tn;
     float g_low, c_low, g_full, c_full;
 };
 
-inline double tile_time(const TileCost& t, int64_t M, int64_t N, int64_t K, int cus) {
+inline double tile_time(const TileCost& t, int64_t M, int64_t N, int64_t K, int cus, double g_min = 0.0) {
     const double tiles = (double)((M + t.tm - 1) / t.tm) * (double)((N + t.tn - 1) / t.tn);
     const double fill = std::min(1.0, tiles / cus);
     const double rounds = t.tm * t.tn <= 64 * 64 && tiles > cus ? tiles / cus + 0.3 : std::ceil(tiles / cus);
-    const double g = t.g_low + (t.g_full - t.g_low) * fill, c = t.c_low + (t.c_full - t.c_low) * fill;
+    const double g = std::max(g_min, t.g_low + (t.g_full - t.g_low) * fill), c = t.c_low + (t.c_full - t.c_low) * fill;
     return 3.0 + rounds * (g + (double)(K / BK) * c);
 }
 
@@ -65,19 +68,25 @@ constexpr double kBigOnce = 4.0;
 // The index of the small tile that a launch takes, or -1 for the 256 x 256
 // tiles. Below O_MIN_KT steps the persistent kernel cannot run. A last stripe
 // of at most TAIL_ROWS rows costs the 256 x 256 tiles no round. Within 3 % of
-// each other the 256 x 256 tiles win.
+// each other the 256 x 256 tiles win. No row/column tile's prologue is taken for
+// shorter than 64 x 64's: the fitted 0.5 us of 256 x 192 for a few tiles, outside
+// the fit at K 128, gave it launches of two workgroups (65 x 128 -> 384 5.3 us,
+// with 64 x 64 tiles 3.0 us); the floor changes no pick from K 256 on.
+constexpr double kPrologueRowcol = 1.3;
 inline int small_plan(int mode, int64_t M, int64_t N, int64_t K, int cus) {
     const bool row = mode == ROWCOL;
     if (M <= TAIL_ROWS && K / BK >= (row ? O_MIN_KT : 4)) return -1;  // the tail kernel alone
     const TileCost* const t = row ? kSmallRowcol : kSmallBlockwise;
     const int count = row ? (int)std::size(kSmallRowcol) : (int)std::size(kSmallBlockwise);
+    const double g_min = row ? kPrologueRowcol : 0.0;
+    auto small_time = [&](int i) { return tile_time(t[i], M, N, K, cus, g_min); };
     int best = 0;
     for (int i = 1; i < count; ++i)
-        if (tile_time(t[i], M, N, K, cus) < tile_time(t[best], M, N, K, cus)) best = i;
+        if (small_time(i) < small_time(best)) best = i;
     if (row && K / BK < O_MIN_KT) return best;
     const int64_t tail = M % BM, Mb = tail <= TAIL_ROWS && M > tail ? M - tail : M;
     const double big = kBigOnce + tile_time(row ? kBigRowcol : kBigBlockwise, Mb, N, K, cus);
-    return tile_time(t[best], M, N, K, cus) < 0.97 * big ? best : -1;
+    return small_time(best) < 0.97 * big ? best : -1;
 }
 
 // A launch's route: small tile `small`, or (small < 0) rows [0, Mt) in 256 x 256
