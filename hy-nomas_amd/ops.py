@@ -79,21 +79,19 @@ def eager_op(name: str, mutates_args=()):
         required = sum(not a.has_default_value() for a in args)
         mutated = [(i, n) for i, n in enumerate(names) if n in mutates_args]
 
-        def direct(v, kind, grad) -> bool:
-            if type(v) not in kind:
-                return False
-            return not isinstance(v, torch.Tensor) or not (
-                (grad and v.requires_grad) or not v.is_cuda or v.is_neg() or v._is_zerotensor())
-
         def plain(pos, kw) -> bool:
             if len(pos) > len(kinds) or (len(pos) < required and any(n not in kw for n in names[len(pos):required])):
                 return False
             grad = torch.is_grad_enabled()
             for v, kind in zip(pos, kinds):
-                if not direct(v, kind, grad):
+                t = type(v)
+                if t not in kind or (t in _TENSOR and (not v.is_cuda or v.is_neg() or v._is_zerotensor()
+                                                       or (grad and v.requires_grad))):
                     return False
             for n, v in kw.items():
-                if not direct(v, by_name.get(n, ()), grad):
+                t = type(v)
+                if t not in by_name.get(n, ()) or (t in _TENSOR and (not v.is_cuda or v.is_neg() or v._is_zerotensor()
+                                                                     or (grad and v.requires_grad))):
                     return False
             try:
                 return not _observed()
