@@ -130,20 +130,20 @@ constexpr int GROUP_M = 8;  // tile rows per group of a queue (L2 reuse of A and
 
 HN_GEMM_HD int imin(int a, int b) { return a < b ? a : b; }
 
-// Tile counts of an M x N output in 256-row, bn-column tiles: whole tiles
-// first (tm_full x tn_full), then the edge tiles (the last row stripe if M %
-// 256 != 0, then the last column stripe if N % bn != 0); per_xcd is the
-// longest XCD queue (each class split evenly over the 8 XCDs).
+// Tile counts of an M x N output in 256 x 256 tiles: whole tiles first
+// (tm_full x tn_full), then the edge tiles (the last row stripe if M % 256 !=
+// 0, then the last column stripe if N % 256 != 0); per_xcd is the longest XCD
+// queue (each class split evenly over the 8 XCDs).
 struct TileCounts {
     int tiles_m, tiles_n, tm_full, tn_full, m_tail, tiles_full, tiles_part, per_xcd;
 };
 
-HN_GEMM_HD TileCounts tile_counts(int64_t M, int64_t N, int bn) {
+HN_GEMM_HD TileCounts tile_counts(int64_t M, int64_t N) {
     TileCounts t;
     t.tiles_m = (int)((M + 255) / 256);
-    t.tiles_n = (int)((N + bn - 1) / bn);
+    t.tiles_n = (int)((N + 255) / 256);
     t.tm_full = (int)(M / 256);
-    t.tn_full = (int)(N / bn);
+    t.tn_full = (int)(N / 256);
     t.m_tail = (int)(M % 256 != 0);
     t.tiles_full = t.tm_full * t.tn_full;
     t.tiles_part = t.tiles_m * t.tiles_n - t.tiles_full;
@@ -246,11 +246,11 @@ struct WaveExtent {
     int imax, jmax;
 };
 
-HN_GEMM_HD WaveExtent wave_extent(int64_t M, int64_t N, int64_t row0, int64_t col0, int wc) {
+HN_GEMM_HD WaveExtent wave_extent(int64_t M, int64_t N, int64_t row0, int64_t col0) {
     const int64_t rows = M - row0, cols = N - col0;
     WaveExtent e;
     e.jmax = rows >= 128 ? 4 : (rows <= 0 ? 0 : (int)((rows + 31) >> 5));
-    e.imax = cols >= wc ? wc / 32 : (cols <= 0 ? 0 : (int)(cols >> 5));
+    e.imax = cols >= 128 ? 4 : (cols <= 0 ? 0 : (int)(cols >> 5));
     return e;
 }
 
@@ -258,15 +258,14 @@ HN_GEMM_HD WaveExtent wave_extent(int64_t M, int64_t N, int64_t row0, int64_t co
 // Output stores of the persistent kernel, also shared with the CPU checker
 // (tests/gemm_tiles_check.cpp walks every store of every wave through these).
 //
-// A wave stores its 128 x wc sub-tile (first row m0w, first column n0w)
+// A wave stores its 128 x 128 sub-tile (first row m0w, first column n0w)
 // through a raw buffer "window": base = element (m0w, n0w), size =
 // out_window_bytes. A store's offset is bytes from the base (row * pitch +
 // 2 * column, pitch = 2 ldc); the buffer's range check drops a store whose
 // offset is at or past the size, i.e. every store to a row at or past M (a
 // store never straddles a row, so never the size). The size is zero when no
-// row or no column block is inside. Columns past N: with wc = 128 and N a
-// multiple of 128 a wave's columns are all inside or none (imax 4 or 0);
-// with wc = 96 each store tests its columns against imax (oe_store_on).
+// row or no column block is inside. Columns past N: N is a multiple of 128, so
+// a wave's columns are all inside or none (imax 4 or 0).
 
 HN_GEMM_HD uint32_t mul24(uint32_t a, uint32_t b) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -291,10 +290,6 @@ HN_GEMM_HD uint32_t oe_store_off(uint32_t pitch, int lane, int P, int q) {
            (uint32_t)(32 * (P >> 1) + 8 * q) * pitch + (uint32_t)(128 * (P & 1));
 }
 
-HN_GEMM_HD bool oe_store_on(int wc, int imax, int P, int lane) {
-    return wc == 128 || 64 * (P & 1) + 8 * (lane & 7) < 32 * imax;
-}
-
 // Row order of the MFMA fragment reads: lane l reads row oe_row(l % 32) of
 // each 32-row block of both operands (bits 2 and 3 exchanged; an involution
 // that maps each aligned group of 16 rows onto itself). The accumulator block
@@ -311,8 +306,6 @@ HN_GEMM_HD uint32_t direct_store_off(uint32_t pitch, int lane, int P, int ii, in
     return mul24((uint32_t)oe_row(lane & 31), pitch) + (uint32_t)(32 * (P >> 1)) * pitch +
            (uint32_t)(2 * (32 * i + 16 * hv + 8 * (lane >> 5)));
 }
-
-HN_GEMM_HD bool direct_store_on(int wc, int imax, int i) { return 32 * i < wc && (wc == 128 || i < imax); }
 
 }  // namespace gemm
 }  // namespace hn

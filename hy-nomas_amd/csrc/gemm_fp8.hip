@@ -428,7 +428,7 @@ constexpr int O_PASSES = 2 * O_JO;                  // overlapped passes (steps 
 static_assert(O_MIN_KT == O_PASSES + 3, "a tile's K steps: the passes, the tail step and the last two");
 static_assert(O_SMEM <= 160 * 1024, "LDS");
 
-// Output window of one wave's 128 x wc sub-tile (first row m0w, first column
+// Output window of one wave's 128 x 128 sub-tile (first row m0w, first column
 // n0w): a raw buffer whose range check drops the stores to rows past M (the
 // store geometry and the window's size are gemm_dma.h's, shared with the CPU
 // checker), so the stores carry no per-lane test and no 64-bit address
@@ -571,19 +571,17 @@ HN_DEVICE uint4 oe_readback(const uint8_t* stg, int q, int lane) {
 }
 
 // Store q of pass P of the pending sub-tile (gemm_dma.h: oe_store_off), through
-// its output window (pimax: its column blocks inside the matrix).
-HN_DEVICE void oe_store(__amdgpu_buffer_rsrc_t win, int pimax, uint32_t pitch, int P, int q, const uint4& v,
-                        int lane) {
-    if (oe_store_on(O_WC, pimax, P, lane))
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), win,
-                                               (int)oe_store_off(pitch, lane, P, q), 0, 0);
+// its output window.
+HN_DEVICE void oe_store(__amdgpu_buffer_rsrc_t win, uint32_t pitch, int P, int q, const uint4& v, int lane) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), win,
+                                           (int)oe_store_off(pitch, lane, P, q), 0, 0);
 }
 
 // All eight passes of a pending tile without overlap (before an edge tile and
 // after a workgroup's last tile).
 template <int ACT>
 HN_DEVICE void oe_flush(const Params& p, uint32_t (&y)[4][4][8], uint8_t* stg, __amdgpu_buffer_rsrc_t win,
-                        int pimax, int lane) {
+                        int lane) {
     const uint32_t pitch = (uint32_t)p.ldc * 2;
 #pragma unroll
     for (int P = 0; P < O_PASSES; ++P) {
@@ -593,7 +591,7 @@ HN_DEVICE void oe_flush(const Params& p, uint32_t (&y)[4][4][8], uint8_t* stg, _
 #pragma unroll
         for (int g = 0; g < 4; ++g) oe_write(y, stg, P, g >> 1, g & 1, lane);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) oe_store(win, pimax, pitch, P, q, oe_readback(stg, q, lane), lane);
+        for (int q = 0; q < 4; ++q) oe_store(win, pitch, P, q, oe_readback(stg, q, lane), lane);
     }
 }
 
@@ -606,7 +604,7 @@ HN_DEVICE void oe_flush(const Params& p, uint32_t (&y)[4][4][8], uint8_t* stg, _
 // rows' 128-byte lines, which the L2 merges.
 template <int ACT>
 HN_DEVICE void direct_passes(const Params& p, const f32x16 (&acc)[4][4], const uint8_t* prm,
-                             __amdgpu_buffer_rsrc_t win, int imax, int lane) {
+                             __amdgpu_buffer_rsrc_t win, int lane) {
     const int h = lane >> 5, r = oe_row(lane & 31);
     const uint32_t pitch = (uint32_t)p.ldc * 2;
 #pragma unroll
@@ -645,12 +643,10 @@ HN_DEVICE void direct_passes(const Params& p, const f32x16 (&acc)[4][4], const u
                 w[2 * vq] = o.x;
                 w[2 * vq + 1] = o.y;
             }
-            if (direct_store_on(O_WC, imax, i)) {
-                __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{w[0], w[1], w[2], w[3]}, win,
-                                                       (int)direct_store_off(pitch, lane, P, ii, 0), 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{w[4], w[5], w[6], w[7]}, win,
-                                                       (int)direct_store_off(pitch, lane, P, ii, 1), 0, 0);
-            }
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{w[0], w[1], w[2], w[3]}, win,
+                                                   (int)direct_store_off(pitch, lane, P, ii, 0), 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{w[4], w[5], w[6], w[7]}, win,
+                                                   (int)direct_store_off(pitch, lane, P, ii, 1), 0, 0);
         }
     }
 }
@@ -822,15 +818,14 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
     auto dma_lane = [&](int l) { return dma_lane_of(wave, l, p.K); };
     auto dma_off = [&](const DmaLane& d, int q, uint32_t lim) { return dma_offset(d, q, p.K, lim); };
     // Current tile: origin and blocks inside the matrix (imax weight blocks of
-    // the wave's wc columns, 4 or 3 in the interior; jmax activation blocks of
-    // 32 rows). Wave-uniform. Tiles with every block inside the matrix take
-    // the carried path.
+    // the wave's 128 columns, jmax activation blocks of 32 rows). Wave-uniform.
+    // Tiles with every block inside the matrix take the carried path.
     int64_t cm0 = 0, cn0 = 0;
     int cimax = 0, cjmax = 0;
     auto set_cur = [&](int tm_, int tn_) {
         cm0 = (int64_t)tm_ * BM;
         cn0 = (int64_t)tn_ * TBN;
-        const WaveExtent e = wave_extent(p.M, p.N, cm0 + wm * 128, cn0 + wn * O_WC, O_WC);
+        const WaveExtent e = wave_extent(p.M, p.N, cm0 + wm * 128, cn0 + wn * O_WC);
         cimax = e.imax;
         cjmax = e.jmax;
     };
@@ -847,10 +842,9 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
     f32x16 acc[4][4];
     i32x8 fa[4], fb[4];
     uint32_t y[4][4][8];         // carried rows (j < O_JO) of the pending tile
-    // Pending tile: its output window and column blocks inside (none yet: an
-    // empty window, every store dropped).
+    // Pending tile: its output window (none yet: an empty window, every store
+    // dropped).
     __amdgpu_buffer_rsrc_t pwin = out_window(p, p.M, 0, 0);
-    int pimax = 0;
     bool pending = false;
 
     // Fragment reads. A fragment of block row base + 32 q is 16-byte chunks
@@ -940,7 +934,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
             // staging writes (slots 3-15), stores two slots after each read.
             if (PASS >= 1 && s < 4) rb[s] = oe_readback(stg, s, el);
             if (PASS >= 1 && s >= 2 && s < 6)
-                oe_store(pwin, pimax, pitch, PASS - 1, s - 2, rb[s - 2], el);
+                oe_store(pwin, pitch, PASS - 1, s - 2, rb[s - 2], el);
             const int i = s >> 2, j = s & 3;
             if (!EDGE || (i < cimax && j < cjmax)) acc[i][j] = mfma(fb[i], fa[j], acc[i][j]);
             if (NEXT) roll(s, an, bnx, 0, rl);
@@ -1031,7 +1025,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
             step(KT - 1, F{}, std::integral_constant<int, -1>{}, std::integral_constant<int, 0>{}, F{}, F{});
             stamp(2);
         } else {
-            if (pending) oe_flush<ACT>(p, y, stg, pwin, pimax, fresh_lane());
+            if (pending) oe_flush<ACT>(p, y, stg, pwin, fresh_lane());
             step(0, T{}, std::integral_constant<int, -1>{}, std::integral_constant<int, 3>{}, T{}, T{});
             for (int k = 1; k < KT - 2; ++k)
                 step(k, T{}, std::integral_constant<int, -1>{}, std::integral_constant<int, 1>{}, T{}, F{});
@@ -1053,12 +1047,11 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
         }
         stamp(4);
         const __amdgpu_buffer_rsrc_t cwin = out_window(p, cm0 + wm * 128, cn0 + wn * O_WC, cimax);
-        direct_passes<ACT>(p, acc, prm, cwin, cimax, fresh_lane());
+        direct_passes<ACT>(p, acc, prm, cwin, fresh_lane());
         stamp(5);
         convert_tile(acc, y, prm, fresh_lane());
         stamp(6);
         pwin = cwin;
-        pimax = cimax;
         pending = true;
         if (!more) break;
         par = (KT + par) & 1;
@@ -1072,7 +1065,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_rowcol_oe_kernel(Params p) {
         ++stamp_tile;
 #endif
     }
-    oe_flush<ACT>(p, y, stg, pwin, pimax, fresh_lane());
+    oe_flush<ACT>(p, y, stg, pwin, fresh_lane());
     // The last step's re-load of step 0 (no next tile) may still be landing.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (p.tail_M > p.M) {

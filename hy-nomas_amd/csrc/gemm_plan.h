@@ -125,7 +125,7 @@ inline Route gemm_route(int mode, int64_t M, int64_t N, int64_t K, int cus, int 
         }
     }
     r.Mt = stripe ? M - m_tail : M;
-    r.tiles = tile_counts(r.Mt, N, BN);
+    r.tiles = tile_counts(r.Mt, N);
     const int per_xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
     const int cap = wg_cap >= 1 && wg_cap < per_xcd_cus ? wg_cap : per_xcd_cus;
     r.S = r.tiles.per_xcd < cap ? r.tiles.per_xcd : cap;

@@ -1,10 +1,10 @@
 // CPU bounds check of the persistent FP8 GEMM's operand loads, built from the
 // kernel's own load geometry (hy-nomas_amd/csrc/gemm_dma.h): for an M x N x K
-// problem with bn-column tiles, every load of every wave, of every tile and
+// problem in 256 x 256 tiles, every load of every wave, of every tile and
 // every K step, of both operands, is checked to stay inside its operand, and
 // loads of rows inside a tile to keep their exact offset.
 //
-// usage: gemm_dma_check M N K bn [nocap]
+// usage: gemm_dma_check M N K [nocap]
 //   nocap: leave the offsets uncapped (the checker must then find loads out
 //          of bounds for a shape whose last tile is partial).
 // Prints "loads=<n> out_of_bounds=<n> wrong_offset=<n>"; exit 0.
@@ -97,7 +97,7 @@ static int tailwide_main(int argc, char** argv) {
         return 2;
     }
     const int64_t Mt = M - M % 256;
-    const TileCounts t = tile_counts(Mt, N, 256);
+    const TileCounts t = tile_counts(Mt, N);
     const Queue q{t.tiles_n, t.tm_full, t.tn_full, t.tiles_full, t.tiles_part, t.m_tail};
     const int per_xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
     const int S = t.per_xcd < per_xcd_cus ? t.per_xcd : per_xcd_cus;
@@ -203,20 +203,20 @@ int main(int argc, char** argv) {
     if (argc > 1 && strcmp(argv[1], "small") == 0) return small_main(argc, argv);
     if (argc > 1 && strcmp(argv[1], "tail") == 0) return tail_main(argc, argv);
     if (argc > 1 && strcmp(argv[1], "tailwide") == 0) return tailwide_main(argc, argv);
-    if (argc < 5) {
-        fprintf(stderr, "usage: %s M N K bn [nocap]\n", argv[0]);
+    if (argc < 4) {
+        fprintf(stderr, "usage: %s M N K [nocap]\n", argv[0]);
         return 2;
     }
-    const int64_t M = atoll(argv[1]), N = atoll(argv[2]), K = atoll(argv[3]), bn = atoll(argv[4]);
-    const bool nocap = argc > 5 && strcmp(argv[5], "nocap") == 0;
-    if (M <= 0 || N <= 0 || K <= 0 || K % 128 || (bn != 256 && bn != 192)) {
+    const int64_t M = atoll(argv[1]), N = atoll(argv[2]), K = atoll(argv[3]);
+    const bool nocap = argc > 4 && strcmp(argv[4], "nocap") == 0;
+    if (M <= 0 || N <= 0 || K <= 0 || K % 128) {
         fprintf(stderr, "bad shape\n");
         return 2;
     }
     long long loads = 0, oob = 0, wrong = 0;
-    const int64_t extents[2] = {M, N}, tiles[2] = {256, bn};
+    const int64_t extents[2] = {M, N}, tile = 256;
     for (int operand = 0; operand < 2; ++operand) {
-        const int64_t extent = extents[operand], tile = tiles[operand];
+        const int64_t extent = extents[operand];
         for (int64_t t0 = 0; t0 < extent; t0 += tile) {
             const int64_t rows = extent - t0 < tile ? extent - t0 : tile;
             const uint32_t lim = nocap ? 0xffffffffu : dma_limit(rows, K);

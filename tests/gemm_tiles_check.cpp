@@ -5,14 +5,14 @@
 // the first entry without a tile) and counts how often each output tile is
 // produced. With STORES = 1 it also walks every store the kernel makes for
 // every tile -- per lane and wave 16 carried stores and 16 direct stores of
-// 16 bytes, with the same header's offsets, predicates and output-window
+// 16 bytes, with the same header's offsets and output-window
 // sizes -- and applies the buffer range check (a store whose offset is at or
 // past the window's size is dropped): each output element inside M x N must
 // be written exactly once, and no store may land outside M x N or outside its
 // own wave's columns, or straddle the window's end. It also checks that each
 // wave's MFMA blocks (wave_extent's imax, jmax) cover all its outputs.
 //
-// Usage: gemm_tiles_check M N BN CUS [LDC STORES]
+// Usage: gemm_tiles_check M N CUS [LDC STORES]
 // Prints: tiles=<count> missing=<n> repeated=<n> out_of_range=<n> max_full=<n>
 //         max_edge=<n> max_load_x100=<100 * max over workgroups of full + edge / 2>
 //         uncovered=<outputs> stores=<kept stores> dropped=<stores>
@@ -31,15 +31,15 @@ struct Queue {
 };
 
 int main(int argc, char** argv) {
-    if (argc != 5 && argc != 7) {
-        fprintf(stderr, "usage: %s M N BN CUS [LDC STORES]\n", argv[0]);
+    if (argc != 4 && argc != 6) {
+        fprintf(stderr, "usage: %s M N CUS [LDC STORES]\n", argv[0]);
         return 2;
     }
     const long long M = atoll(argv[1]), N = atoll(argv[2]);
-    const int bn = atoi(argv[3]), cus = atoi(argv[4]);
-    const long long ldc = argc == 7 ? atoll(argv[5]) : N;
-    const bool walk_stores = argc == 7 && atoi(argv[6]) != 0;
-    const TileCounts t = tile_counts(M, N, bn);
+    const int cus = atoi(argv[3]);
+    const long long ldc = argc == 6 ? atoll(argv[4]) : N;
+    const bool walk_stores = argc == 6 && atoi(argv[5]) != 0;
+    const TileCounts t = tile_counts(M, N);
     const Queue q{t.tiles_n, t.tm_full, t.tn_full, t.tiles_full, t.tiles_part, t.m_tail};
     const int per_xcd_cus = cus / 8 > 0 ? cus / 8 : 1;
     const int S = t.per_xcd < per_xcd_cus ? t.per_xcd : per_xcd_cus;  // the launch's grid / 8
@@ -47,7 +47,7 @@ int main(int argc, char** argv) {
     std::vector<unsigned char> writes(walk_stores ? (size_t)(M * N) : 0, 0);
     int max_full = 0, max_edge = 0, max_load = 0, bad = 0;
     long long uncovered = 0, kept = 0, dropped = 0, outside = 0, straddle = 0;
-    const int wc = bn / 2;
+    const int wc = 128;
     const uint32_t pitch = (uint32_t)(ldc * 2);
     // One store of `bytes` bytes at offset `off` of the window of the wave at
     // (row0, col0) whose size is `size`.
@@ -72,8 +72,8 @@ int main(int argc, char** argv) {
     auto check_waves = [&](int tm, int tn) {
         for (int wm = 0; wm < 2; ++wm)
             for (int wn = 0; wn < 2; ++wn) {
-                const long long row0 = (long long)tm * 256 + wm * 128, col0 = (long long)tn * bn + wn * wc;
-                const WaveExtent e = wave_extent(M, N, row0, col0, wc);
+                const long long row0 = (long long)tm * 256 + wm * 128, col0 = (long long)tn * 256 + wn * wc;
+                const WaveExtent e = wave_extent(M, N, row0, col0);
                 for (int r = 0; r < 128; ++r)
                     for (int c = 0; c < wc; ++c) {
                         const bool valid = row0 + r < M && col0 + c < N;
@@ -84,13 +84,11 @@ int main(int argc, char** argv) {
                 for (int lane = 0; lane < 64; ++lane) {
                     for (int P = 0; P < 4; ++P)  // carried passes (or their flush)
                         for (int qq = 0; qq < 4; ++qq)
-                            if (oe_store_on(wc, e.imax, P, lane))
-                                store(row0, col0, size, oe_store_off(pitch, lane, P, qq), 16);
+                            store(row0, col0, size, oe_store_off(pitch, lane, P, qq), 16);
                     for (int P = 4; P < 8; ++P)  // direct passes
                         for (int ii = 0; ii < 2; ++ii)
                             for (int hv = 0; hv < 2; ++hv)
-                                if (direct_store_on(wc, e.imax, 2 * (P & 1) + ii))
-                                    store(row0, col0, size, direct_store_off(pitch, lane, P, ii, hv), 16);
+                                store(row0, col0, size, direct_store_off(pitch, lane, P, ii, hv), 16);
                 }
             }
     };

@@ -29,8 +29,8 @@ def checker(tmp_path_factory):
     return exe
 
 
-def _run(exe, M, N, bn, cus=256, ldc=None, stores=False):
-    args = [str(exe), str(M), str(N), str(bn), str(cus)]
+def _run(exe, M, N, cus=256, ldc=None, stores=False):
+    args = [str(exe), str(M), str(N), str(cus)]
     if stores:
         args += [str(ldc or N), "1"]
     out = subprocess.run(args, check=True, capture_output=True, text=True).stdout
@@ -42,18 +42,17 @@ def _stores_ok(r):
             and r["stores"] > 0)
 
 
-@pytest.mark.parametrize("M,N,bn", [
-    (10800, 12288, 256), (10800, 3072, 256), (10800, 9216, 256), (10800, 4096, 256), (10800, 12288 + 64, 256),
-    (4096, 3072, 192), (132, 12288, 256), (132, 3072, 192), (4996, 3072, 256), (1, 128, 256),
-    (300, 640, 256), (257, 257, 256), (10752, 12288, 256), (8192, 8192, 256), (5000, 7000, 256),
-    (65536, 1024, 256), (100, 256, 192), (100, 256, 256), (227, 1024, 256), (97, 384, 192),
+@pytest.mark.parametrize("M,N", [
+    (10800, 12288), (10800, 3072), (10800, 9216), (10800, 4096), (10800, 12288 + 64), (4096, 3072), (132, 12288),
+    (132, 3072), (4996, 3072), (1, 128), (300, 640), (257, 257), (10752, 12288), (8192, 8192), (5000, 7000),
+    (65536, 1024), (100, 256), (227, 1024), (97, 384),
 ])
 @pytest.mark.parametrize("cus", [256, 80])
-def test_every_tile_exactly_once(checker, M, N, bn, cus):
+def test_every_tile_exactly_once(checker, M, N, cus):
     # the stores are walked once per shape, for the GEMM's N (a multiple of
     # 128; 257 and 7000 only exercise the queues)
     stores = cus == 256 and N % 128 == 0
-    r = _run(checker, M, N, bn, cus, stores=stores)
+    r = _run(checker, M, N, cus, stores=stores)
     assert r["missing"] == 0 and r["repeated"] == 0 and r["out_of_range"] == 0, r
     if N % 128 == 0:
         # each wave's MFMA blocks cover all its outputs
@@ -62,24 +61,23 @@ def test_every_tile_exactly_once(checker, M, N, bn, cus):
         assert _stores_ok(r), r
 
 
-@pytest.mark.parametrize("M,N,bn", [(100, 256, 192), (227, 1024, 256), (10752 + 100, 3072, 256), (48, 640, 256)])
-def test_rows_past_m_are_dropped_by_the_window(checker, M, N, bn):
+@pytest.mark.parametrize("M,N", [(100, 256), (227, 1024), (10752 + 100, 3072), (48, 640)])
+def test_rows_past_m_are_dropped_by_the_window(checker, M, N):
     """Waves with fewer than 128 rows left (97..127 of them among these
     shapes: four row blocks, some rows past M) store whole 128-row sub-tiles;
     the window drops the stores past M and every output is still written
     once. Taking four row blocks for a whole sub-tile once let stores past row
     M through (a GPU memory fault at M = 100)."""
-    r = _run(checker, M, N, bn, stores=True)
+    r = _run(checker, M, N, stores=True)
     assert r["dropped"] > 0 and _stores_ok(r), r
 
 
-@pytest.mark.parametrize("M,N,bn,ldc", [(300, 640, 256, 648), (300, 384, 192, 392), (130, 256, 256, 1 << 22),
-                                        (97, 384, 192, 1 << 22)])
-def test_row_pitch_past_n(checker, M, N, bn, ldc):
+@pytest.mark.parametrize("M,N,ldc", [(300, 640, 648), (300, 384, 392), (130, 256, 1 << 22), (97, 384, 1 << 22)])
+def test_row_pitch_past_n(checker, M, N, ldc):
     """ldc > N: the stores keep to the first N columns of each row, up to the
     largest pitch the GEMM accepts (2^22 columns, 128 rows of which still fit
     the 32-bit offsets)."""
-    r = _run(checker, M, N, bn, ldc=ldc, stores=True)
+    r = _run(checker, M, N, ldc=ldc, stores=True)
     assert _stores_ok(r), r
 
 
@@ -95,7 +93,7 @@ def test_a_full_window_is_caught(tmp_path):
                                                       f'#include "{HERE.parent}/hy-nomas_amd/csrc/gemm_dma.h"'))
     subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", str(tmp_path / "planted.cpp"), "-o", str(exe)],
                    check=True)
-    r = _run(exe, 100, 256, 256, stores=True)
+    r = _run(exe, 100, 256, stores=True)
     assert r["store_outside"] > 0, r
 
 
@@ -104,5 +102,5 @@ def test_edge_tiles_go_to_the_shorter_queues(checker, M, N, full_rounds):
     # 10800 rows: a 48-row last tile row. The longest queue holds full_rounds
     # full tiles; the edge tiles (half-cost in this count) land on the
     # workgroups with one full tile fewer, so no queue exceeds full_rounds.
-    r = _run(checker, M, N, 256)
+    r = _run(checker, M, N)
     assert r["max_full"] == full_rounds and r["max_load_x100"] == 100 * full_rounds, r
