@@ -429,9 +429,10 @@ HN_DEVICE void store_tile(const CacheRegs<NW>& r, uint8_t* st, const float* sb) 
 // Unquantized tail tile (bf16 K/V of the current chunk), written with the
 // same thread-to-location mapping as the cache writes (so it cleanly
 // replaces what those wrote to the same stage). The loads and the LDS writes
-// are separate steps: the 8-wave loop issues a tail tile's loads one tile
-// ahead, as it does a cache tile's, into TailRegs; the 4-wave loop (two
-// stages, registers already near the limit) loads and writes in one go.
+// are separate steps: the tail loops of both shapes, and the 8-wave general
+// loop, issue a tail tile's loads ahead into TailRegs, as they do a cache
+// tile's; the 4-wave general loop (which holds a cache tile's prefetch beside
+// it, near the register limit) loads and writes in one go (copy_tail_k / _v).
 template <int NW>
 struct TailRegs {
     uint4 k[2 * Shape<NW>::KU];        // unit i: dims 16 u .. + 7 in k[2 i], + 8 .. + 15 in k[2 i + 1]
@@ -951,8 +952,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
     // fetched are cache tiles -- the bulk of any long range. They run a loop
     // with no per-tile geometry, tail or mask branches, loading through
     // descriptors that span the (b, h) cache rows [0, cache_end) at the
-    // tile's byte offset (so the span must fit 31 bits). Kernels with
-    // validity masks take the general loop throughout.
+    // tile's byte offset (so the span must fit 31 bits). The MASK
+    // instantiations run it too: a tile's validity word then masks its blocks
+    // (mask_word). The tiles up to the tail take the general loop in both
+    // instantiations, the tail's tiles a loop of their own where tail_span holds.
     const int64_t full_end = cache_end < wg_key_limit ? cache_end : wg_key_limit;
     const int n_full = full_end > 0 ? (int)(full_end / BKV) : 0;
     const bool span_ok = cache_end > 0 && p.cs1 > 0 && p.ss1 > 0 &&
@@ -980,7 +983,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_fp8kv_kernel(Params p) {
     //           scales of t + NS to buffer (u + NS) % 2, V codes fetched
     // NS = 2 (the loop below, written for it): K of t + 1 is written in half
     // 0 and read by S(t + 1) in half 1, so a barrier ends half 0 as well as
-    // the tile. NS = 3 (the generic loop after it): every tile a half
+    // the tile. NS = 3 (the loops after it): every tile a half
     // reads was written before the barrier that ended an earlier tile, and
     // the stage written during tile t (that of t - 1) was last read in half 1
     // of t - 1, before the barrier ending it; one barrier per tile.

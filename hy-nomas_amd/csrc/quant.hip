@@ -152,8 +152,8 @@ __global__ __launch_bounds__(256) void quantize_rows_wide_kernel(
 //
 // RES: x is first the block's gated residual, x <- bf16(x + bf16(y * gate[b]))
 // (bf16 tensor ops of nomas_compile_prepost.py:75-88), written to `out`. As
-// separate kernels the product, the sum and the LayerNorm read or write 8 bf16
-// rows and one row of codes; here 3 and one: 10800 x 3072 89 -> 58 us.
+// separate kernels the product (2), the sum (3) and the LayerNorm (1) read or
+// write 6 bf16 rows and one row of codes; here 3 and one: 10800 x 3072 89 -> 58 us.
 // `out` may be x itself (each wave stores a row it has loaded), so x is not
 // __restrict__ in the kernels that take a Residual.
 struct Residual {
@@ -447,9 +447,6 @@ __global__ void status_clear_kernel(int32_t* status) {
     if (threadIdx.x == 0) *status = 0;
 }
 
-// One (batch, token, head) row of 128 bf16 per 16-lane group, 8 per lane, in
-// a grid-stride loop; rows are walked token-fastest when the source's token
-// stride is the smaller one, so that consecutive groups read adjacent rows.
 constexpr int KV_ROWS_PER_GROUP = 4;  // rows each 16-lane group carries (loads issued together)
 constexpr int KV_UNIT = 16 * KV_ROWS_PER_GROUP;
 
@@ -458,7 +455,8 @@ constexpr int KV_UNIT = 16 * KV_ROWS_PER_GROUP;
 // [B, H, L, D] source viewed as [B, L, H, D]): the loads of consecutive rows
 // are then consecutive 256-byte rows of the source, and each 128-byte code row
 // is still one whole cache line.
-// Row k of group g (16 lanes) in a unit, k = 0..3. TOKEN_FAST: token 8 tt + g % 8
+//
+// kv_unit_row: row k of group g (16 lanes) in a unit, k = 0..3. TOKEN_FAST: token 8 tt + g % 8
 // of heads 8 ht + 4 (g / 8) + k -- for each k the loads are two runs of 8
 // consecutive tokens (2 KB each), and every token's 8 heads of codes (1 KB) and
 // scales (one 32-byte sector) are written by the unit. Otherwise rows g + 16 k
