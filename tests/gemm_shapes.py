@@ -105,8 +105,8 @@ SMALL_BLOCKWISE = {
     (2000, 4096, 1024): "128x256",
     (1300, 3200, 640): "128x256",
 }
-# One shape per accumulation: 64 x 64 adds each K block's product by its factor;
-# the others carry the accumulators in units of the block's factor.
+# One shape per kernel: 64 x 64 and 128 x 128 add each K block's product by its
+# factor; 128 x 256 and 256 x 256 carry the accumulators in units of the block's.
 ZERO_FACTORS = {
     (300, 384, 1024): "64x64",
     (1000, 2048, 1024): "128x128",

@@ -326,8 +326,8 @@ def test_blockwise_gemm_zero_block_factors(O, dev, m, n, k):
 def test_blockwise_gemm_factor_jump_of_2_to_60(O, dev, direction, m, n, k):
     """Adjacent K blocks whose weight factors differ by 2^60, the widest span
     the FP8Linear loader accepts: the carried accumulator's rescale by
-    f_prev / f (2^60 or 2^-60 here; 64 x 64 tiles have none) stays finite, and
-    the result matches the float64 dequantize-then-matmul reference."""
+    f_prev / f (2^60 or 2^-60 here; 128 x 256 and 256 x 256 tiles) stays finite,
+    and the result matches the float64 dequantize-then-matmul reference."""
     print(f"case blockwise factor jump {direction} {m}x{n}x{k}", flush=True)
     pf = pkg_module("pixelumm_fp8")
     g = torch.Generator().manual_seed(31)
