@@ -261,6 +261,27 @@ def test_direct_calls_need_the_private_names_of_torch(monkeypatch):
     assert ops._stream(torch.zeros(1)) == 7
 
 
+def test_rules_registered_on_an_op_are_met(monkeypatch):
+    """The registration methods of torch.library's custom ops stay on the ops, and an op
+    that a program has registered something on is called through the dispatcher."""
+    ops = pkg_module("ops")
+    for name in ("register_autograd", "register_vmap", "register_kernel", "register_torch_dispatch",
+                 "set_kernel_enabled", "register_fake"):
+        assert callable(getattr(ops.linear_fp8, name)), name
+
+    class Plain:
+        pass
+
+    ran = []
+    monkeypatch.setitem(ops._KINDS, "Tensor", (Plain,))
+    monkeypatch.setattr(torch.library, "custom_op", lambda name, fn, mutates_args: _FakeOp(ran))
+    op = ops.eager_op("test::op")(lambda x: ran.append("direct"))
+    op(Plain())
+    op.register_autograd("rule")
+    op(Plain())
+    assert ran == ["direct", "register_autograd rule", "op"]
+
+
 @pytest.mark.parametrize("owner,name", [("autograd.forward_ad", "_current_level"), ("_C", "_len_torch_dispatch_stack"),
                                         ("autograd", "_profiler_enabled"), ("_C", "_cuda_getCurrentRawStream")])
 def test_ops_load_without_a_private_name_of_torch(owner, name):
@@ -279,6 +300,9 @@ class _FakeOp:
         arg = type("A", (), {"name": "x", "type": "Tensor", "has_default_value": lambda self: False})()
         self._opoverload = type("O", (), {"_schema": type("S", (), {"arguments": [arg]})})
         self.register_fake = None
+
+    def register_autograd(self, rule):
+        self.ran.append(f"register_autograd {rule}")
 
     def __call__(self, x):
         self.ran.append("op")
