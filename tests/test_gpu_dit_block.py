@@ -481,6 +481,36 @@ def test_block_with_text_compiled_is_eager(dev):
     assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
 
 
+def test_denoising_pass_in_a_graph(dev):
+    """A denoising pass with text recorded into a graph: every replay on new inputs, with
+    eager work between the replays, gives the eager call's bits."""
+    print("case dit block graph", flush=True)
+    blk, (img, txt, vec, cos, sin, cache, hist), masks = _text_block(dev, 47)
+
+    def call():
+        return blk(img, vec, cos, sin, cache, hist, txt=txt, vec_txt=vec, **masks)
+
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(2):
+                call()
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = call()
+        g = torch.Generator(device=dev).manual_seed(48)
+        for _ in range(3):
+            for t in (img, txt, vec):
+                t.copy_(torch.randn(t.shape, device=dev, generator=g))
+            graph.replay()
+            torch.cuda.synchronize()
+            ref = call()
+            torch.cuda.synchronize()
+            assert torch.equal(out[0], ref[0]) and torch.equal(out[1], ref[1])
+
+
 def test_compiled_update_of_the_cached_attention(dev):
     """The seam's write pass, compiled: the eager pass's outputs,
     cache and mask bits, and a non-finite value is refused."""
