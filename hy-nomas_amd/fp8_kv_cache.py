@@ -104,8 +104,10 @@ def read_flag_later(status: torch.Tensor):
     was refused. Work enqueued in between keeps the GPU busy: waiting for the
     word at once drains the stream, and the host then enqueues behind an idle
     GPU (about 170 us in a block's write pass). A compiled caller reads the word
-    at once: pinned memory and events do not trace (inductor refuses both)."""
-    if torch.compiler.is_compiling():
+    at once: pinned memory and events do not trace (inductor refuses both). So
+    does a capturing stream, where a read is refused at this place, before an
+    event of the capture is left with the pinned-memory allocator."""
+    if torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing():
         _raise_if_flagged(status)
         return lambda: None
     word = torch.empty(1, dtype=torch.int32, pin_memory=True)

@@ -89,3 +89,12 @@ def test_write_verdict_under_compile_is_read_at_once():
     with pytest.raises(ValueError, match="non-finite"):
         compiled(torch.ones(1, dtype=torch.int32), torch.ones(2))
     torch._dynamo.reset()
+
+
+def test_write_verdict_on_a_capturing_stream_is_read_at_once(monkeypatch):
+    """No pinned memory and no event there: the plain read, which a capture refuses."""
+    kvc = pkg_module("fp8_kv_cache")
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    kvc.read_flag_later(torch.zeros(1, dtype=torch.int32))()
+    with pytest.raises(ValueError, match="non-finite"):
+        kvc.read_flag_later(torch.ones(1, dtype=torch.int32))
